@@ -57,8 +57,9 @@ struct ZS16 {
   f16x2 s;   // scale twice
 };
 struct ZSbf {
-  float z;
-  float s;
+  f16x2 zb;  // (1024 + z) twice
+  f16x2 zh;  // -(64 + z) twice
+  float s;   // scale
 };
 
 // (a & mask) | bits.  gfx9 VOP3 encodings (v_and_or_b32) take no literal
@@ -75,14 +76,21 @@ __device__ __forceinline__ uint32_t opaque_vgpr(uint32_t v) {
   return v;
 }
 
-// Loop-invariant dequantisation constants, held in VGPRs (see and_or).
+// The value v, hidden from constant folding and held in an SGPR.
+__device__ __forceinline__ uint32_t opaque_sgpr(uint32_t v) {
+  asm volatile("" : "+s"(v));
+  return v;
+}
+
+// Loop-invariant dequantisation constants, held in registers (see and_or).
 struct DqK {
   uint32_t lo;     // 0x000F000F: nibbles 0 and 4 of a word
   uint32_t hi;     // 0x00F000F0: nibbles 1 and 5
   uint32_t magic;  // 0x64006400: the fp16 pair (1024, 1024)
+  uint32_t nzero;  // fp32 -0 (the bf16 path's addend)
 };
 __device__ __forceinline__ DqK dq_consts() {
-  return DqK{opaque_vgpr(0x000F000Fu), opaque_vgpr(0x00F000F0u), opaque_vgpr(0x64006400u)};
+  return DqK{opaque_vgpr(0x000F000Fu), opaque_vgpr(0x00F000F0u), opaque_vgpr(0x64006400u), opaque_sgpr(0x80000000u)};
 }
 
 // Typed load at a 32-bit byte offset from a uniform base pointer, so the
@@ -100,75 +108,92 @@ __device__ __forceinline__ T ld_off_nt(const void* base, uint32_t byte_off) {
 template <typename DT>
 struct Dq;
 
-// fp16, per 32-bit word (pairs i = rows (2i, 2i+1) = nibbles (i, i + 4)):
+// Constant pairs of a zero point for q_minus_z.
+__device__ __forceinline__ void zero_pairs(uint32_t z, f16x2& zb, f16x2& zh) {
+  const uint32_t b = 0x6400u | z;
+  const uint32_t h = 0xD400u | (z << 4);
+  zb = __builtin_bit_cast(f16x2, b | (b << 16));
+  zh = __builtin_bit_cast(f16x2, h | (h << 16));
+}
+
+// The integers q - z of one 32-bit word as four fp16 pairs (pair i = rows
+// (2i, 2i+1) = nibbles (i, i + 4)):
 //   nibbles 0,4:  w & 0x000F000F | 0x64006400   = the pair (1024 + q)
 //   nibbles 1,5:  w & 0x00F000F0 | 0x64006400   = the pair (1024 + 16 q)
 //   nibbles 2,6 and 3,7: the same on w >> 8.
 // (1024 + q) - (1024 + z) and fma(1024 + 16 q, 1/16, -(64 + z)) are both the
-// exact integer q - z (fp16 integers below 2048, power-of-two scaling), and
-// the one packed multiply by the scale is the single round-to-nearest-even
-// of (q - z) * s that the oracle specifies: 13 VALU operations per word.
+// exact integer q - z (fp16 integers below 2048, power-of-two scaling): 9 VALU
+// operations per word.
+__device__ __forceinline__ void q_minus_z(uint32_t w, f16x2 zb, f16x2 zh, const DqK& k, f16x2 (&d)[4]) {
+  const f16x2 inv16 = __builtin_bit_cast(f16x2, 0x2C002C00u);  // (1/16, 1/16)
+  const uint32_t w8 = w >> 8;
+  d[0] = __builtin_bit_cast(f16x2, and_or(w, k.lo, k.magic)) - zb;
+  d[1] = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, and_or(w, k.hi, k.magic)), inv16, zh);
+  d[2] = __builtin_bit_cast(f16x2, and_or(w8, k.lo, k.magic)) - zb;
+  d[3] = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, and_or(w8, k.hi, k.magic)), inv16, zh);
+}
+
+// fp16: the one packed multiply of q - z by the scale is the single
+// round-to-nearest-even of (q - z) * s that the oracle specifies: 13 VALU
+// operations per word.
 template <>
 struct Dq<F16> {
   using ZS = ZS16;
+  static constexpr int kOps = 13;  // vector operations of word()
   __device__ __forceinline__ static ZS make(uint32_t z, uint16_t sbits) {
     ZS r;
-    const uint32_t zb = 0x6400u | z;
-    const uint32_t zh = 0xD400u | (z << 4);
-    r.zb = __builtin_bit_cast(f16x2, zb | (zb << 16));
-    r.zh = __builtin_bit_cast(f16x2, zh | (zh << 16));
+    zero_pairs(z, r.zb, r.zh);
     r.s = __builtin_bit_cast(f16x2, (uint32_t)sbits | ((uint32_t)sbits << 16));
     return r;
   }
   __device__ __forceinline__ static f16x8 word(uint32_t w, const ZS& zs, const DqK& k) {
-    const f16x2 inv16 = __builtin_bit_cast(f16x2, 0x2C002C00u);  // (1/16, 1/16)
-    const uint32_t w8 = w >> 8;
-    const f16x2 a0 = __builtin_bit_cast(f16x2, and_or(w, k.lo, k.magic));
-    const f16x2 a1 = __builtin_bit_cast(f16x2, and_or(w, k.hi, k.magic));
-    const f16x2 a2 = __builtin_bit_cast(f16x2, and_or(w8, k.lo, k.magic));
-    const f16x2 a3 = __builtin_bit_cast(f16x2, and_or(w8, k.hi, k.magic));
-    const f16x2 h0 = (a0 - zs.zb) * zs.s;
-    const f16x2 h1 = __builtin_elementwise_fma(a1, inv16, zs.zh) * zs.s;
-    const f16x2 h2 = (a2 - zs.zb) * zs.s;
-    const f16x2 h3 = __builtin_elementwise_fma(a3, inv16, zs.zh) * zs.s;
-    const u32x4 r = {__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1),
-                     __builtin_bit_cast(uint32_t, h2), __builtin_bit_cast(uint32_t, h3)};
+    f16x2 d[4];
+    q_minus_z(w, zs.zb, zs.zh, k, d);
+    const u32x4 r = {__builtin_bit_cast(uint32_t, d[0] * zs.s), __builtin_bit_cast(uint32_t, d[1] * zs.s),
+                     __builtin_bit_cast(uint32_t, d[2] * zs.s), __builtin_bit_cast(uint32_t, d[3] * zs.s)};
     return __builtin_bit_cast(f16x8, r);
   }
   // The exact integers q - z (no scaling): 9 VALU operations per word, for
   // kernels that apply the group scale to the fp32 sums instead.
   __device__ __forceinline__ static f16x8 word_q_minus_z(uint32_t w, const ZS& zs, const DqK& k) {
-    const f16x2 inv16 = __builtin_bit_cast(f16x2, 0x2C002C00u);  // (1/16, 1/16)
-    const uint32_t w8 = w >> 8;
-    const f16x2 h0 = __builtin_bit_cast(f16x2, and_or(w, k.lo, k.magic)) - zs.zb;
-    const f16x2 h1 = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, and_or(w, k.hi, k.magic)), inv16, zs.zh);
-    const f16x2 h2 = __builtin_bit_cast(f16x2, and_or(w8, k.lo, k.magic)) - zs.zb;
-    const f16x2 h3 = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, and_or(w8, k.hi, k.magic)), inv16, zs.zh);
-    const u32x4 r = {__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1),
-                     __builtin_bit_cast(uint32_t, h2), __builtin_bit_cast(uint32_t, h3)};
+    f16x2 d[4];
+    q_minus_z(w, zs.zb, zs.zh, k, d);
+    const u32x4 r = {__builtin_bit_cast(uint32_t, d[0]), __builtin_bit_cast(uint32_t, d[1]),
+                     __builtin_bit_cast(uint32_t, d[2]), __builtin_bit_cast(uint32_t, d[3])};
     return __builtin_bit_cast(f16x8, r);
   }
 };
 
-// bf16: (q - z) * s is exact in fp32 (4-bit by 8-bit significands) and the
-// conversion to bf16 is the single round-to-nearest-even.
+// bf16: q - z as exact fp16 pairs, times the fp32 scale by one v_fma_mix_f32
+// per weight (the product of a 5-bit integer and an 8-bit significand is
+// exact; adding -0 keeps the product's sign of zero), and the conversion to
+// bf16 is the single round-to-nearest-even: 21 VALU operations per word, where
+// unpacking each nibble to fp32 by itself (extract, convert, subtract,
+// multiply) took 36.  The vector work bounds the bf16 kernels that dequantise
+// once per few rows: E = 128, H = 2048, I = 768 top-8 experts in bf16 405 ->
+// 277 us for three blocks at 24 tokens and 865 -> 685 us for one at 4096; the
+// Llama-3-8B linears at M = 8192 3246 -> 2969 us.  (Scaling the biased pairs
+// 1024 + q by one FMA with addend -(1024 + z) s would take 17, but loses the
+// sign of an infinite scale's products.)
 template <>
 struct Dq<BF16> {
   using ZS = ZSbf;
+  static constexpr int kOps = 21;
   __device__ __forceinline__ static ZS make(uint32_t z, uint16_t sbits) {
     ZS r;
-    r.z = (float)z;
+    zero_pairs(z, r.zb, r.zh);
     r.s = __builtin_bit_cast(float, (uint32_t)sbits << 16);
     return r;
   }
-  __device__ __forceinline__ static bf16x8 word(uint32_t w, const ZS& zs, const DqK&) {
+  __device__ __forceinline__ static bf16x8 word(uint32_t w, const ZS& zs, const DqK& k) {
+    const float nz = __builtin_bit_cast(float, k.nzero);
+    f16x2 d[4];
+    q_minus_z(w, zs.zb, zs.zh, k, d);
     bf16x8 r;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float lo = (float)((w >> (4 * i)) & 0xFu);
-      const float hi = (float)((w >> (4 * i + 16)) & 0xFu);
-      r[2 * i] = (__bf16)((lo - zs.z) * zs.s);
-      r[2 * i + 1] = (__bf16)((hi - zs.z) * zs.s);
+      r[2 * i] = (__bf16)__builtin_fmaf((float)d[i][0], zs.s, nz);
+      r[2 * i + 1] = (__bf16)__builtin_fmaf((float)d[i][1], zs.s, nz);
     }
     return r;
   }

@@ -303,7 +303,7 @@ __global__ __launch_bounds__(64 * WN * WK) void gemv_kernel(
 
   // ---- compute ---------------------------------------------------------------
   // bf16 (not biased): per k-block the weights are dequantised to (q - z) * s
-  // with the oracle's rounding (Dq<DT>::word, 13 VALU operations per 8
+  // with the oracle's rounding (Dq<DT>::word, 21 VALU operations per 8
   // weights) into the MFMA A operand, accumulated in fp32; fp16 takes the
   // integers q - z (9 operations) and scales each k-tile's sum in fp32.
   // Biased path (GEMMs of up to 3 rows, where the vector work of dequantising

@@ -466,14 +466,14 @@ __device__ __forceinline__ void moe_pass(const MoeArgs& a, u32x4* __restrict__ x
 #pragma unroll
         for (int j = 0; j < TW; ++j) acc[mt][j] = mfma16x16x32(av[cur][j], bx[cur][mt], acc[mt][j]);
       if (w + 1 < 4) {
-        // MC * TW MFMAs, MC LDS reads and 13 * TW vector operations (TW
+        // MC * TW MFMAs, MC LDS reads and kOps * TW vector operations (TW
         // words' dequantisation) per k-block: spread the reads and the
         // vector work between the MFMAs.
 #pragma unroll
         for (int i = 0; i < MC * TW; ++i) {
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                 // MFMA
           if (i < MC) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);     // LDS read
-          __builtin_amdgcn_sched_group_barrier(0x002, (13 * TW + MC * TW - 1) / (MC * TW), 0);  // VALU
+          __builtin_amdgcn_sched_group_barrier(0x002, (Dq<DT>::kOps * TW + MC * TW - 1) / (MC * TW), 0);  // VALU
         }
         __builtin_amdgcn_sched_barrier(0);
       }

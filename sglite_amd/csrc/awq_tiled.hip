@@ -39,6 +39,8 @@
 // Replaces awq_gemm_kernel / awq_gemm_triton
 // (python/sglite/srt/model_executor/layers/quantization/awq_triton.py:16-195)
 // and gptq_marlin_gemm (marlin_utils.py:388-410) for large batches.
+#include <type_traits>
+
 #include "awq_buffer.h"
 #include "awq_device.h"
 #include "awq_epilogue.h"
@@ -320,7 +322,7 @@ __global__ __launch_bounds__(256) void tiled_kernel(TiledArgs a) {
   };
   // The MFMAs of one block, with the LDS reads and dequantisation of the
   // next block spread between them (one LDS read, then four MFMAs each
-  // followed by up to two VALU operations, per m-tile).
+  // followed by two VALU operations, three in bf16, per m-tile).
   auto mma = [&](int slot) {
 #pragma unroll
     for (int mt = 0; mt < MTL; ++mt)
@@ -332,7 +334,7 @@ __global__ __launch_bounds__(256) void tiled_kernel(TiledArgs a) {
 #pragma unroll
       for (int r = 0; r < NTW; ++r) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-        __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
+        __builtin_amdgcn_sched_group_barrier(0x002, (Dq<DT>::kOps + 7) / 8, 0);  // VALU
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -796,14 +798,14 @@ __global__ __launch_bounds__(64 * NW, OCC) void mfma32_kernel(TiledArgs a) {
 #pragma unroll
         for (int g = 0; g < 2; ++g) acc[i][g] = mfma32x32x16(av[cur][g], bx[cur][i], acc[i][g]);
       if (st + 1 < NST) {
-        // 2 MT MFMAs, MT LDS reads and 26 vector operations (two words'
+        // 2 MT MFMAs, MT LDS reads and 2 kOps vector operations (two words'
         // dequantisation) per step: after each MFMA one LDS read (while
-        // there are any) and up to four vector operations.
+        // there are any) and four vector operations, six in bf16.
 #pragma unroll
         for (int i = 0; i < 2 * MT; ++i) {
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
           if (i < MT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
-          __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // VALU
+          __builtin_amdgcn_sched_group_barrier(0x002, (Dq<DT>::kOps + 3) / 4, 0);  // VALU
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -1015,6 +1017,10 @@ hipError_t launch_bm(const TiledArgs& a, int gpt, hipStream_t s) {
 
 template <typename DT>
 hipError_t launch_dt(const GemmPlan& p, const TiledArgs& a, int gpt, hipStream_t s) {
+  // The bf16 32-row form is cut for three workgroups per CU: at four (128
+  // registers) its dequantisation spills 57 registers inside the loop
+  // (Qwen3-4B decode linears at M = 32: 77 us a layer, 61.6 at three).
+  constexpr int kOcc32 = std::is_same_v<DT, BF16> ? 3 : 4;
   switch (p.variant) {
     case 32: return launch_bm<32, DT>(a, gpt, s);
     case 64: return launch_bm<64, DT>(a, gpt, s);
@@ -1023,7 +1029,7 @@ hipError_t launch_dt(const GemmPlan& p, const TiledArgs& a, int gpt, hipStream_t
     case 1128: return launch_bm32<128, 3, 1, 4, DT>(a, gpt, s);
     case 2064: return launch_bm32<64, 3, 2, 4, DT>(a, gpt, s);
     case 2128: return launch_bm32<128, 2, 2, 4, DT>(a, gpt, s);
-    case 4032: return launch_bm32<32, 3, 4, 4, DT>(a, gpt, s);
+    case 4032: return launch_bm32<32, 3, kOcc32, 4, DT>(a, gpt, s);
     case 8064: return launch_bm32<64, 3, 1, 8, DT>(a, gpt, s);
     case 8128: return launch_bm32<128, 3, 1, 8, DT>(a, gpt, s);
     case 9064: return launch_bm32<64, 3, 1, 8, DT, 2>(a, gpt, s);

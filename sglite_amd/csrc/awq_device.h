@@ -82,15 +82,14 @@ __device__ __forceinline__ uint32_t opaque_sgpr(uint32_t v) {
   return v;
 }
 
-// Loop-invariant dequantisation constants, held in registers (see and_or).
+// Loop-invariant dequantisation constants, held in VGPRs (see and_or).
 struct DqK {
   uint32_t lo;     // 0x000F000F: nibbles 0 and 4 of a word
   uint32_t hi;     // 0x00F000F0: nibbles 1 and 5
   uint32_t magic;  // 0x64006400: the fp16 pair (1024, 1024)
-  uint32_t nzero;  // fp32 -0 (the bf16 path's addend)
 };
 __device__ __forceinline__ DqK dq_consts() {
-  return DqK{opaque_vgpr(0x000F000Fu), opaque_vgpr(0x00F000F0u), opaque_vgpr(0x64006400u), opaque_sgpr(0x80000000u)};
+  return DqK{opaque_vgpr(0x000F000Fu), opaque_vgpr(0x00F000F0u), opaque_vgpr(0x64006400u)};
 }
 
 // Typed load at a 32-bit byte offset from a uniform base pointer, so the
@@ -147,10 +146,18 @@ struct Dq<F16> {
     return r;
   }
   __device__ __forceinline__ static f16x8 word(uint32_t w, const ZS& zs, const DqK& k) {
-    f16x2 d[4];
-    q_minus_z(w, zs.zb, zs.zh, k, d);
-    const u32x4 r = {__builtin_bit_cast(uint32_t, d[0] * zs.s), __builtin_bit_cast(uint32_t, d[1] * zs.s),
-                     __builtin_bit_cast(uint32_t, d[2] * zs.s), __builtin_bit_cast(uint32_t, d[3] * zs.s)};
+    const f16x2 inv16 = __builtin_bit_cast(f16x2, 0x2C002C00u);  // (1/16, 1/16)
+    const uint32_t w8 = w >> 8;
+    const f16x2 a0 = __builtin_bit_cast(f16x2, and_or(w, k.lo, k.magic));
+    const f16x2 a1 = __builtin_bit_cast(f16x2, and_or(w, k.hi, k.magic));
+    const f16x2 a2 = __builtin_bit_cast(f16x2, and_or(w8, k.lo, k.magic));
+    const f16x2 a3 = __builtin_bit_cast(f16x2, and_or(w8, k.hi, k.magic));
+    const f16x2 h0 = (a0 - zs.zb) * zs.s;
+    const f16x2 h1 = __builtin_elementwise_fma(a1, inv16, zs.zh) * zs.s;
+    const f16x2 h2 = (a2 - zs.zb) * zs.s;
+    const f16x2 h3 = __builtin_elementwise_fma(a3, inv16, zs.zh) * zs.s;
+    const u32x4 r = {__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1),
+                     __builtin_bit_cast(uint32_t, h2), __builtin_bit_cast(uint32_t, h3)};
     return __builtin_bit_cast(f16x8, r);
   }
   // The exact integers q - z (no scaling): 9 VALU operations per word, for
@@ -172,7 +179,7 @@ struct Dq<F16> {
 // multiply) took 36.  The vector work bounds the bf16 kernels that dequantise
 // once per few rows: E = 128, H = 2048, I = 768 top-8 experts in bf16 405 ->
 // 277 us for three blocks at 24 tokens and 865 -> 685 us for one at 4096; the
-// Llama-3-8B linears at M = 8192 3246 -> 2969 us.  (Scaling the biased pairs
+// Llama-3-8B linears at M = 8192 3369 -> 3029 us.  (Scaling the biased pairs
 // 1024 + q by one FMA with addend -(1024 + z) s would take 17, but loses the
 // sign of an infinite scale's products.)
 template <>
@@ -186,7 +193,10 @@ struct Dq<BF16> {
     return r;
   }
   __device__ __forceinline__ static bf16x8 word(uint32_t w, const ZS& zs, const DqK& k) {
-    const float nz = __builtin_bit_cast(float, k.nzero);
+    // fp32 -0, the addend.  Made here and not once per kernel: the asm keeps one word's operations
+    // together.  Without it the scheduler spreads the words of a k-tile, and
+    // the 128-row forms spill 32 to 50 registers (8 to 57 at 32 rows).
+    const float nz = __builtin_bit_cast(float, opaque_sgpr(0x80000000u));
     f16x2 d[4];
     q_minus_z(w, zs.zb, zs.zh, k, d);
     bf16x8 r;

@@ -1017,9 +1017,9 @@ hipError_t launch_bm(const TiledArgs& a, int gpt, hipStream_t s) {
 
 template <typename DT>
 hipError_t launch_dt(const GemmPlan& p, const TiledArgs& a, int gpt, hipStream_t s) {
-  // The bf16 32-row form is cut for three workgroups per CU: at four (128
-  // registers) its dequantisation spills 57 registers inside the loop
-  // (Qwen3-4B decode linears at M = 32: 77 us a layer, 61.6 at three).
+  // The bf16 32-row form is cut for three workgroups per CU (141 registers):
+  // at four it would spill inside the loop (Qwen3-4B decode linears at M = 32:
+  // 77 us a layer with 57 spilled registers, 58.8 at three workgroups).
   constexpr int kOcc32 = std::is_same_v<DT, BF16> ? 3 : 4;
   switch (p.variant) {
     case 32: return launch_bm<32, DT>(a, gpt, s);

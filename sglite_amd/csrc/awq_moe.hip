@@ -793,6 +793,16 @@ hipError_t launch_moe_align(const int32_t* ids, int64_t n, int64_t E, int64_t bs
 }
 
 hipError_t launch_moe_gemm(const MoeGemmParams& p, hipStream_t s) {
+  // At most one routed row per expert on average: the row-block form, whose
+  // grid is the blocks that have rows.  Here most experts are empty, and the
+  // grid below, sized for every expert being busy, leaves the rest of a token's
+  // 8 experts to 32 workgroups (E = 128, H = 2048, I = 768 top-8 fp16 / bf16, a
+  // block's whole forward: T = 1 56.7 -> 28.4 / 67.4 -> 29.2 us, T = 8 69.9 ->
+  // 58.5 / 82.6 -> 62.3, T = 16 81.5 -> 73.4 / 96.2 -> 78.5; beyond that line
+  // it loses: T = 32 84.7 -> 90.2, and E = 64, H = 2048, I = 1408 at T = 16
+  // 82.7 -> 83.4).  Its per-expert weight offsets are 32 bits, past-the-end
+  // offsets bit 31.
+  if (p.num_routed <= p.E && p.g.NT * p.g.KT * 1024 < (int64_t(1) << 31)) return launch_moe_rows(p, s);
   MoeArgs a{};
   a.x = p.x;
   a.x_bytes = (uint32_t)((p.num_routed + p.a_div - 1) / p.a_div * p.g.K * 2);

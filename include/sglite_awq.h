@@ -42,7 +42,7 @@ enum {
   AWQ_STATUS_WORKSPACE = -4         /* workspace missing or too small          */
 };
 
-enum { AWQ_DTYPE_FP16 = 0, AWQ_DTYPE_BF16 = 1 };
+enum { AWQ_DTYPE_FP16 = 0, AWQ_DTYPE_BF16 = 1, AWQ_DTYPE_FP32 = 2 /* router logits only */ };
 
 /* Message of the last failed call on this thread ("" if none). */
 const char* awq_last_error(void);
@@ -343,6 +343,14 @@ int64_t awq_moe_block_capacity(int64_t numel, int64_t E, int64_t block_size);
 int awq_moe_align_block_size(const int32_t* topk_ids, int64_t numel, int64_t E, int64_t block_size,
                              int32_t* sorted_ids, int32_t* expert_ids, int32_t* num_tokens_post_pad,
                              int32_t* expert_offsets, awq_stream_t stream);
+
+/* awq_moe_topk_softmax and awq_moe_align_block_size of the same tokens, the
+ * logits in fp16, bf16 or fp32 (dtype AWQ_DTYPE_FP16, AWQ_DTYPE_BF16,
+ * AWQ_DTYPE_FP32), in one launch for a decode batch.  T >= 1; outputs and
+ * limits are those of the two. */
+int awq_moe_route(const void* gating_output, int dtype, int64_t T, int64_t E, int64_t topk, int renormalize,
+                  int64_t block_size, float* topk_weights, int32_t* topk_ids, int32_t* sorted_ids,
+                  int32_t* expert_ids, int32_t* num_tokens_post_pad, int32_t* expert_offsets, awq_stream_t stream);
 
 enum { AWQ_MOE_ACT_NONE = 0, AWQ_MOE_ACT_SILU = 1, AWQ_MOE_ACT_GELU = 2 };
 

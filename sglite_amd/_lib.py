@@ -22,6 +22,7 @@ AWQ_STATUS_WORKSPACE = -4
 
 AWQ_DTYPE_FP16 = 0
 AWQ_DTYPE_BF16 = 1
+AWQ_DTYPE_FP32 = 2  # router logits only
 
 _vp = ctypes.c_void_p
 _i64 = ctypes.c_int64
@@ -68,6 +69,7 @@ SIGNATURES = {
     "awq_moe_sorted_capacity": (_i64, [_i64, _i64, _i64]),
     "awq_moe_block_capacity": (_i64, [_i64, _i64, _i64]),
     "awq_moe_align_block_size": (_int, [_vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp]),
+    "awq_moe_route": (_int, [_vp, _int, _i64, _i64, _i64, _int, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "awq_moe_w4a16_gemm": (_int, [_vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _i64, _vp, _vp, _i64,
                                   _i64, _int, _int, _vp, _vp]),
     "awq_moe_sum_reduce": (_int, [_vp, _vp, _i64, _i64, _i64, _int, _vp]),

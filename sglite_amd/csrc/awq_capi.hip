@@ -645,6 +645,31 @@ int awq_moe_align_block_size(const int32_t* topk_ids, int64_t numel, int64_t E, 
                     "awq_moe_align_block_size launch");
 }
 
+int awq_moe_route(const void* gating_output, int dtype, int64_t T, int64_t E, int64_t topk, int renormalize,
+                  int64_t block_size, float* topk_weights, int32_t* topk_ids, int32_t* sorted_ids,
+                  int32_t* expert_ids, int32_t* num_tokens_post_pad, int32_t* expert_offsets, awq_stream_t stream) {
+  const TraceRange range("awq_moe_route");
+  if (dtype != AWQ_DTYPE_FP16 && dtype != AWQ_DTYPE_BF16 && dtype != AWQ_DTYPE_FP32)
+    return fail(AWQ_STATUS_INVALID_ARGUMENT, "awq_moe_route: dtype must be 0, 1 or 2, got %d", dtype);
+  if (E <= 0 || E > 512)
+    return fail(AWQ_STATUS_UNSUPPORTED, "awq_moe_route: E must be in [1, 512], got %lld", (long long)E);
+  if (topk < 1 || topk > E || topk > 64)
+    return fail(AWQ_STATUS_INVALID_ARGUMENT, "awq_moe_route: topk must be in [1, min(E, 64)], got %lld",
+                (long long)topk);
+  if (T < 1 || T * topk >= (int64_t(1) << 24))
+    return fail(AWQ_STATUS_UNSUPPORTED, "awq_moe_route: T must be at least 1 and T * topk below 2^24");
+  if (block_size <= 0 || block_size % 16 != 0 || block_size > 1024)
+    return fail(AWQ_STATUS_INVALID_ARGUMENT,
+                "awq_moe_route: block_size must be a positive multiple of 16 up to 1024, got %lld",
+                (long long)block_size);
+  if (!gating_output || !topk_weights || !topk_ids || !sorted_ids || !expert_ids || !num_tokens_post_pad ||
+      !expert_offsets)
+    return fail(AWQ_STATUS_INVALID_ARGUMENT, "awq_moe_route: null pointer argument");
+  const MoeRouteParams p{gating_output, dtype, T, E, topk, block_size, renormalize ? 1 : 0, topk_weights, topk_ids,
+                         sorted_ids, expert_ids, num_tokens_post_pad, expert_offsets};
+  return hip_status(launch_moe_route(p, (hipStream_t)stream), "awq_moe_route launch");
+}
+
 int awq_moe_w4a16_gemm(const void* a, int64_t a_rows, const void* w, const void* s, const void* z, int64_t E,
                        int64_t N, int64_t K, int64_t G, int dtype, const int32_t* sorted_ids, int64_t sorted_cap,
                        const int32_t* expert_offsets, const float* topk_weights, int64_t num_routed, int64_t top_k,

@@ -98,6 +98,21 @@ hipError_t launch_moe_topk(const float* logits, float* tw, int32_t* tid, int64_t
 hipError_t launch_moe_align(const int32_t* ids, int64_t n, int64_t E, int64_t bs, int32_t* sorted, int32_t* expert_ids,
                             int32_t* num_post_pad, int32_t* offsets, hipStream_t s);
 
+// Routing and alignment together (in one launch for a decode batch).
+struct MoeRouteParams {
+  const void* logits;  // [T, E]
+  int dtype;           // of the logits: 0 fp16, 1 bf16, 2 fp32
+  int64_t T, E, k, bs;
+  int renorm;
+  float* tw;           // as launch_moe_topk writes them
+  int32_t* tid;
+  int32_t* sorted;     // as launch_moe_align writes them
+  int32_t* expert_ids;
+  int32_t* num_post_pad;
+  int32_t* offsets;
+};
+hipError_t launch_moe_route(const MoeRouteParams& p, hipStream_t s);
+
 struct MoeGemmParams {
   const void* x;           // activation rows
   const void* w;           // expert-stacked repacked weights / scales / zeros

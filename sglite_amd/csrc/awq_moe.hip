@@ -73,19 +73,15 @@ __device__ __forceinline__ uint64_t lanes_below(int lane) { return lane == 0 ? 0
 // One wave per token; lane l holds experts l, l + 64, ...
 // Follows fused.py:11-31 (topk_softmax, then w / (sum(w) + 1e-8)).
 // ---------------------------------------------------------------------------
-template <int EPL>
-__global__ __launch_bounds__(256) void topk_softmax_kernel(const float* __restrict__ logits, float* __restrict__ tw,
-                                                           int32_t* __restrict__ tid, int T, int E, int k,
-                                                           int renorm) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int t = blockIdx.x * 4 + wave;
-  if (t >= T) return;
-  const float* row = logits + (int64_t)t * E;
+// L: the logits' type, converted to fp32 as they are read.
+template <int EPL, typename L>
+__device__ __forceinline__ void topk_token(const L* __restrict__ row, int lane, int E, int k, int renorm, float& w,
+                                           int& id) {
   float v[EPL];
 #pragma unroll
   for (int i = 0; i < EPL; ++i) {
     const int e = lane + 64 * i;
-    v[i] = e < E ? row[e] : -INFINITY;
+    v[i] = e < E ? (float)row[e] : -INFINITY;
   }
   float mx = v[0];
 #pragma unroll
@@ -127,10 +123,23 @@ __global__ __launch_bounds__(256) void topk_softmax_kernel(const float* __restri
     }
     wsum += top;
   }
+  w = renorm ? wsel / (wsum + 1e-8f) : wsel;
+  id = isel;
+}
+
+template <int EPL, typename L>
+__global__ __launch_bounds__(256) void topk_softmax_kernel(const L* __restrict__ logits, float* __restrict__ tw,
+                                                           int32_t* __restrict__ tid, int T, int E, int k,
+                                                           int renorm) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int t = blockIdx.x * 4 + wave;
+  if (t >= T) return;
+  float w;
+  int id;
+  topk_token<EPL>(logits + (int64_t)t * E, lane, E, k, renorm, w, id);
   if (lane < k) {
-    const float w = renorm ? wsel / (wsum + 1e-8f) : wsel;
     tw[(int64_t)t * k + lane] = w;
-    tid[(int64_t)t * k + lane] = isel;
+    tid[(int64_t)t * k + lane] = id;
   }
 }
 
@@ -160,17 +169,25 @@ constexpr int kAlignWaves = kAlignThreads / 64;
 constexpr int kMaxExperts = 512;
 constexpr int kAlignBatch = 4;  // 64-row groups a wave holds in registers per pass over its rows
 
-__global__ __launch_bounds__(kAlignThreads) void align_kernel(const int32_t* __restrict__ ids, int n, int E, int bs,
-                                                              int32_t* __restrict__ sorted, int32_t* __restrict__ expert_ids,
-                                                              int blocks_cap, int32_t* __restrict__ num_post_pad,
-                                                              int32_t* __restrict__ offsets) {
+struct AlignLds {
   // Per wave and expert: the wave's row count, then its first free position.
-  __shared__ int wpos[kAlignWaves][kMaxExperts];
+  int wpos[kAlignWaves][kMaxExperts];
   // Per wave and expert: the lanes of the current 64-row group with that expert.
-  __shared__ uint64_t wmask[kAlignWaves][kMaxExperts];
-  __shared__ int cnt[kMaxExperts];
-  __shared__ int off[kMaxExperts + 1];
-  __shared__ int wtot[kAlignWaves];
+  uint64_t wmask[kAlignWaves][kMaxExperts];
+  int cnt[kMaxExperts];
+  int off[kMaxExperts + 1];
+  int wtot[kAlignWaves];
+};
+
+__device__ __forceinline__ void align_rows(AlignLds& lds, const int32_t* __restrict__ ids, int n, int E, int bs,
+                                           int32_t* __restrict__ sorted, int32_t* __restrict__ expert_ids,
+                                           int blocks_cap, int32_t* __restrict__ num_post_pad,
+                                           int32_t* __restrict__ offsets) {
+  auto& wpos = lds.wpos;
+  auto& wmask = lds.wmask;
+  auto& cnt = lds.cnt;
+  auto& off = lds.off;
+  auto& wtot = lds.wtot;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int chunk = ((n + kAlignWaves - 1) / kAlignWaves + 63) & ~63;
   const int r0 = min(n, wave * chunk), r1 = min(n, r0 + chunk);
@@ -270,6 +287,48 @@ __global__ __launch_bounds__(kAlignThreads) void align_kernel(const int32_t* __r
       }
     }
   }
+}
+
+__global__ __launch_bounds__(kAlignThreads) void align_kernel(const int32_t* __restrict__ ids, int n, int E, int bs,
+                                                              int32_t* __restrict__ sorted, int32_t* __restrict__ expert_ids,
+                                                              int blocks_cap, int32_t* __restrict__ num_post_pad,
+                                                              int32_t* __restrict__ offsets) {
+  __shared__ AlignLds lds;
+  align_rows(lds, ids, n, E, bs, sorted, expert_ids, blocks_cap, num_post_pad, offsets);
+}
+
+// Routing and alignment of a decode batch in one launch: each wave of one
+// workgroup routes a token and the same workgroup aligns the ids, which it
+// keeps in LDS.  A launch of a captured step costs about 1 us beyond its work,
+// so one token per wave is the line: a block of E = 128, H = 2048, I = 768
+// top-8 experts (fp16, whole forward) takes 26.5 us at T = 1 with it and 27.2
+// with two launches (28.4 with the logits' conversion a third), 74.3 and 73.8
+// at T = 16, 86.6 and 83.8 at T = 32, where the waves route two tokens in turn.
+constexpr int kRouteTokens = kAlignWaves;
+constexpr int kRouteRows = kRouteTokens * 64;  // the ids in LDS (at most 64 experts per token)
+
+template <int EPL, typename L>
+__global__ __launch_bounds__(kAlignThreads) void route_kernel(const L* __restrict__ logits, int T, int E, int k,
+                                                              int renorm, int bs, float* __restrict__ tw,
+                                                              int32_t* __restrict__ tid, int32_t* __restrict__ sorted,
+                                                              int32_t* __restrict__ expert_ids, int blocks_cap,
+                                                              int32_t* __restrict__ num_post_pad,
+                                                              int32_t* __restrict__ offsets) {
+  __shared__ AlignLds lds;
+  __shared__ int32_t ids[kRouteRows];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (const int t = wave; t < T) {
+    float w;
+    int id;
+    topk_token<EPL>(logits + (int64_t)t * E, lane, E, k, renorm, w, id);
+    if (lane < k) {
+      tw[t * k + lane] = w;
+      tid[t * k + lane] = id;
+      ids[t * k + lane] = id;
+    }
+  }
+  __syncthreads();
+  align_rows(lds, ids, T * k, E, bs, sorted, expert_ids, blocks_cap, num_post_pad, offsets);
 }
 
 // ---------------------------------------------------------------------------
@@ -775,14 +834,52 @@ MoeStrides moe_expert_strides(const Geom& g) {
 int64_t moe_sorted_capacity(int64_t n, int64_t E, int64_t bs) { return n + E * (bs - 1); }
 int64_t moe_block_capacity(int64_t n, int64_t E, int64_t bs) { return (moe_sorted_capacity(n, E, bs) + bs - 1) / bs; }
 
+namespace {
+
+template <typename L>
+hipError_t launch_topk_t(const L* logits, float* tw, int32_t* tid, int64_t T, int64_t E, int64_t k, int renorm,
+                         hipStream_t s) {
+  const dim3 grid((unsigned)((T + 3) / 4));
+#define SGL_TOPK(EPL_) \
+  hipLaunchKernelGGL((topk_softmax_kernel<EPL_, L>), grid, dim3(256), 0, s, logits, tw, tid, (int)T, (int)E, (int)k, renorm)
+  if (E <= 64) SGL_TOPK(1);
+  else if (E <= 128) SGL_TOPK(2);
+  else if (E <= 256) SGL_TOPK(4);
+  else SGL_TOPK(8);
+#undef SGL_TOPK
+  return hipGetLastError();
+}
+
+template <typename L>
+hipError_t launch_route_t(const MoeRouteParams& p, const L* logits, hipStream_t s) {
+  const int64_t n = p.T * p.k;
+  if (p.T > kRouteTokens) {
+    const hipError_t e = launch_topk_t(logits, p.tw, p.tid, p.T, p.E, p.k, p.renorm, s);
+    return e != hipSuccess ? e : launch_moe_align(p.tid, n, p.E, p.bs, p.sorted, p.expert_ids, p.num_post_pad, p.offsets, s);
+  }
+#define SGL_ROUTE(EPL_)                                                                                          \
+  hipLaunchKernelGGL((route_kernel<EPL_, L>), dim3(1), dim3(kAlignThreads), 0, s, logits, (int)p.T, (int)p.E,    \
+                     (int)p.k, p.renorm, (int)p.bs, p.tw, p.tid, p.sorted, p.expert_ids,                         \
+                     (int)moe_block_capacity(n, p.E, p.bs), p.num_post_pad, p.offsets)
+  if (p.E <= 64) SGL_ROUTE(1);
+  else if (p.E <= 128) SGL_ROUTE(2);
+  else if (p.E <= 256) SGL_ROUTE(4);
+  else SGL_ROUTE(8);
+#undef SGL_ROUTE
+  return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t launch_moe_topk(const float* logits, float* tw, int32_t* tid, int64_t T, int64_t E, int64_t k, int renorm,
                            hipStream_t s) {
-  const dim3 grid((unsigned)((T + 3) / 4));
-  if (E <= 64) hipLaunchKernelGGL((topk_softmax_kernel<1>), grid, dim3(256), 0, s, logits, tw, tid, (int)T, (int)E, (int)k, renorm);
-  else if (E <= 128) hipLaunchKernelGGL((topk_softmax_kernel<2>), grid, dim3(256), 0, s, logits, tw, tid, (int)T, (int)E, (int)k, renorm);
-  else if (E <= 256) hipLaunchKernelGGL((topk_softmax_kernel<4>), grid, dim3(256), 0, s, logits, tw, tid, (int)T, (int)E, (int)k, renorm);
-  else hipLaunchKernelGGL((topk_softmax_kernel<8>), grid, dim3(256), 0, s, logits, tw, tid, (int)T, (int)E, (int)k, renorm);
-  return hipGetLastError();
+  return launch_topk_t(logits, tw, tid, T, E, k, renorm, s);
+}
+
+hipError_t launch_moe_route(const MoeRouteParams& p, hipStream_t s) {
+  if (p.dtype == 0) return launch_route_t(p, (const _Float16*)p.logits, s);
+  if (p.dtype == 1) return launch_route_t(p, (const __bf16*)p.logits, s);
+  return launch_route_t(p, (const float*)p.logits, s);
 }
 
 hipError_t launch_moe_align(const int32_t* ids, int64_t n, int64_t E, int64_t bs, int32_t* sorted, int32_t* expert_ids,

@@ -77,23 +77,33 @@ def fused_experts_impl(hidden_states: torch.Tensor, w1: AWQMoeWeights, w2: AWQMo
                        apply_router_weight_on_input: bool = False) -> torch.Tensor:
     """Run alignment, both grouped GEMMs and the top-k sum; writes into ``hidden_states``
     and returns it, as fused.py:101-202 does."""
+    _check_experts(hidden_states, w1, w2, activation)
+    assert topk_weights.shape == topk_ids.shape, "topk shape mismatch"
+    T, top_k = hidden_states.shape[0], topk_ids.shape[1]
+    if T * top_k == 0:
+        return hidden_states
+    config = get_default_config(T, w1.num_experts, w1.output_size, w1.input_size, top_k)
+    align = ops.moe_align_block_size(topk_ids.to(torch.int32), config["BLOCK_SIZE_M"], w1.num_experts)
+    return _run_experts(hidden_states, w1, w2, topk_weights, top_k, align, activation, apply_router_weight_on_input)
+
+
+def _check_experts(hidden_states: torch.Tensor, w1: AWQMoeWeights, w2: AWQMoeWeights, activation: str) -> None:
     if activation not in ("silu", "gelu"):
         raise ValueError(f"unsupported activation {activation!r}")
     assert hidden_states.shape[1] == w1.input_size, "Hidden size mismatch"
-    assert topk_weights.shape == topk_ids.shape, "topk shape mismatch"
     assert hidden_states.is_contiguous(), "Hidden_states must be contiguous"
     assert hidden_states.dtype in (torch.float16, torch.bfloat16)
     assert w1.num_experts == w2.num_experts, "expert counts differ"
     assert w2.input_size == w1.output_size // 2, "w2's input size must be half of w1's output size"
     assert w2.output_size == hidden_states.shape[1], "w2's output size must equal the hidden size"
+
+
+def _run_experts(hidden_states: torch.Tensor, w1: AWQMoeWeights, w2: AWQMoeWeights, topk_weights: torch.Tensor,
+                 top_k: int, align: ops.MoeAlignment, activation: str,
+                 apply_router_weight_on_input: bool) -> torch.Tensor:
+    """Both grouped GEMMs over aligned rows and the top-k sum, into ``hidden_states``."""
     T, H = hidden_states.shape
-    top_k = topk_ids.shape[1]
-    E = w1.num_experts
     num_routed = T * top_k
-    if num_routed == 0:
-        return hidden_states
-    config = get_default_config(T, E, w1.output_size, w1.input_size, top_k)
-    align = ops.moe_align_block_size(topk_ids.to(torch.int32), config["BLOCK_SIZE_M"], E)
     # First GEMM: gate/up, routed row r reads token r // top_k; act(gate) * up
     # fused into the epilogue (intermediate_cache1 -> intermediate_cache2).
     cache2 = ops.moe_gemm(hidden_states, w1.experts, w1.input_size, w1.output_size, w1.group_size, align, topk_weights,
@@ -121,6 +131,13 @@ class AWQFusedMoe(BaseMoeBackend):
     def forward(self, hidden_states: torch.Tensor, w1: AWQMoeWeights, w2: AWQMoeWeights, gating_output: torch.Tensor,
                 topk: int, renormalize: bool, activation: str = "silu",
                 apply_router_weight_on_input: bool = False) -> torch.Tensor:
+        T, E = gating_output.shape
+        if T > 0 and hidden_states.shape[0] == T and E == w1.num_experts:
+            _check_experts(hidden_states, w1, w2, activation)
+            config = get_default_config(T, E, w1.output_size, w1.input_size, topk)
+            topk_weights, _, align = ops.moe_route(gating_output, topk, renormalize, config["BLOCK_SIZE_M"])
+            return _run_experts(hidden_states, w1, w2, topk_weights, topk, align, activation,
+                                apply_router_weight_on_input)
         topk_weights, topk_ids = fused_topk(hidden_states=hidden_states, gating_output=gating_output, topk=topk,
                                             renormalize=renormalize)
         return fused_experts_impl(hidden_states, w1, w2, topk_weights, topk_ids, activation,

@@ -835,6 +835,53 @@ def moe_align_block_size(topk_ids: torch.Tensor, block_size: int, num_experts: i
     return MoeAlignment(*torch.ops.sglite_awq.awq_moe_align_block_size(topk_ids, block_size, num_experts))
 
 
+_LOGITS_CODE = {torch.float16: _lib.AWQ_DTYPE_FP16, torch.bfloat16: _lib.AWQ_DTYPE_BF16,
+                torch.float32: _lib.AWQ_DTYPE_FP32}
+
+
+@torch.library.custom_op(f"{NAMESPACE}::awq_moe_route", mutates_args=(), device_types="cuda")
+def _route_op(gating_output: torch.Tensor, topk: int, renormalize: bool, block_size: int) -> Tuple[
+        torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
+    if gating_output.dtype not in _LOGITS_CODE:
+        gating_output = gating_output.float()
+    logits = _aligned(gating_output, 4)
+    T, E = logits.shape
+    dev = logits.device
+    w = torch.empty((T, topk), dtype=torch.float32, device=dev)
+    ids = torch.empty((T, topk), dtype=torch.int32, device=dev)
+    cap, bcap = _align_caps(T * topk, E, block_size)
+    sorted_ids = torch.empty(cap, dtype=torch.int32, device=dev)
+    expert_ids = torch.empty(bcap, dtype=torch.int32, device=dev)
+    npp = torch.empty(1, dtype=torch.int32, device=dev)
+    offsets = torch.empty(E + 1, dtype=torch.int32, device=dev)
+    with _on_device(dev):
+        _lib.check(_lib.load().awq_moe_route(logits.data_ptr(), _LOGITS_CODE[logits.dtype], T, E, topk,
+                                             1 if renormalize else 0, block_size, w.data_ptr(), ids.data_ptr(),
+                                             sorted_ids.data_ptr(), expert_ids.data_ptr(), npp.data_ptr(),
+                                             offsets.data_ptr(), _stream(dev)), "awq_moe_route")
+    return w, ids, sorted_ids, expert_ids, npp, offsets
+
+
+@_route_op.register_fake
+def _(gating_output, topk, renormalize, block_size):
+    T, E = gating_output.shape
+    cap, bcap = _align_caps(T * topk, E, block_size)
+    i32 = [gating_output.new_empty(n, dtype=torch.int32) for n in (cap, bcap, 1, E + 1)]
+    return (gating_output.new_empty((T, topk), dtype=torch.float32),
+            gating_output.new_empty((T, topk), dtype=torch.int32), *i32)
+
+
+def moe_route(gating_output: torch.Tensor, topk: int, renormalize: bool,
+              block_size: int) -> Tuple[torch.Tensor, torch.Tensor, MoeAlignment]:
+    """:func:`moe_topk_softmax` and :func:`moe_align_block_size` of the same tokens (at least one), the logits
+    read in their own dtype."""
+    _require_cuda(gating_output)
+    if gating_output.dim() != 2 or gating_output.shape[0] == 0:
+        raise ValueError("gating_output must be [T, E] with T >= 1")
+    w, ids, *align = torch.ops.sglite_awq.awq_moe_route(gating_output, topk, bool(renormalize), block_size)
+    return w, ids, MoeAlignment(*align)
+
+
 _ACT_CODE = {None: _lib.AWQ_MOE_ACT_NONE, "silu": _lib.AWQ_MOE_ACT_SILU, "gelu": _lib.AWQ_MOE_ACT_GELU}
 _ACT_NAME = {"none": None, "silu": "silu", "gelu": "gelu"}
 
@@ -920,5 +967,5 @@ def moe_sum_reduce(inp: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
 REGISTERED_OPS: List[str] = [
     "awq_repack_cdna4", "awq_unrepack_cdna4", "awq_dequant", "awq_dequant_repacked", "awq_w4a16_gemm",
     "awq_w4a16_gemm_out", "awq_w4a16_gemm_act", "awq_w4a16_gemm_act_out", "awq_repack_experts",
-    "awq_moe_topk_softmax", "awq_moe_align_block_size", "awq_moe_w4a16_gemm", "awq_moe_sum_reduce",
+    "awq_moe_topk_softmax", "awq_moe_align_block_size", "awq_moe_route", "awq_moe_w4a16_gemm", "awq_moe_sum_reduce",
 ]

@@ -60,3 +60,22 @@ def test_row_blocks_match_oracle(T, E, k, K, N, G, bs, routing, activation, mul,
     valid = ids.reshape(-1) >= 0
     err = (out[valid].float() - ref[valid].float()).abs().max().item()
     assert err <= 4 * EPS[dtype] * ref[valid].float().abs().max().item()
+
+
+@pytest.mark.parametrize("T,E,k", [(1, 1, 1), (1, 64, 8), (15, 200, 6), (16, 65, 4), (16, 512, 64), (17, 128, 8),
+                                   (200, 60, 4)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("renorm", [True, False])
+def test_route_matches_its_two_stages(T, E, k, dtype, renorm):
+    """One launch or two, 16-bit logits or fp32: the ids, weights and layout of the separate entry points."""
+    from sglite_amd import ops
+
+    logits = torch.randn((T, E), generator=torch.Generator().manual_seed(T * E + k)).to(dtype).to(DEV)
+    w, ids, align = ops.moe_route(logits, k, renorm, 16)
+    rw, rids = ops.moe_topk_softmax(logits.float(), k, renorm)
+    ref = ops.moe_align_block_size(rids, 16, E)
+    assert torch.equal(w, rw) and torch.equal(ids, rids)
+    total = int(ref.num_tokens_post_pad.item())
+    assert torch.equal(align.sorted_ids[:total], ref.sorted_ids[:total])
+    for got, want in zip(align[1:], ref[1:]):
+        assert torch.equal(got, want)

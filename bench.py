@@ -548,7 +548,7 @@ def pmc_summary(fetch_dir: str, write_dir: str) -> str:
     algo = defaultdict(list)
     for M in M_SET:
         for _, K, N in LAYER:
-            algo[ops.plan_info(M, N, K, G).function].append(gemm_bytes(M, N, K))
+            algo[launched(ops, M, N, K).function].append(gemm_bytes(M, N, K))
     lines = [
         "# HBM traffic of the decode kernels (Qwen3-4B layer, M = 1, 8, 32), rocprofv3 PMC",
         "",
@@ -675,8 +675,21 @@ def bounds_bench(ops, dev: torch.device, reps: int = 7) -> dict:
     return out
 
 
-def _launches_per_call(ops, M: int, N: int, K: int, activation=None) -> int:
+def launched(ops, M: int, N: int, K: int, activation=None):
+    """The plan with the kernel that the launch runs: ring_kernel's grid and k-slices where it takes the place
+    of the planned kernel (17-64 rows)."""
     info = ops.plan_info(M, N, K, G, activation)
+    if not info.ring:
+        return info
+    ntw, wn, wk = info.ring // 10000 % 10, info.ring // 100 % 10, info.ring % 100
+    tiles = (N + 15) // 16
+    groups = -(-tiles // (wn * ntw)) if activation is None else -(-(tiles // 2) // (wn * ntw // 2))
+    return info._replace(function="ring_kernel", variant=info.ring, k_slices=info.ring_slices,
+                         workgroups=groups * info.ring_slices, threads=64 * wn * wk)
+
+
+def _launches_per_call(ops, M: int, N: int, K: int, activation=None) -> int:
+    info = launched(ops, M, N, K, activation)
     return 2 if info.kernel == "tiled_kernel" and info.k_slices > 1 and not info.fixup else 1
 
 
@@ -712,7 +725,8 @@ def sq_workload(ops, dev: torch.device, gen: torch.Generator) -> None:
         x = torch.randn((M, K), generator=gen, device=dev).to(torch.float16)
         out = torch.empty((M, N), dtype=torch.float16, device=dev)
         for _ in range(1 + SQ_REPS):
-            ops.gemm(x, r, K, N, G, counters=cnt, out=out)
+            with ops.plan_overrides(ring=0):  # the planned kernels, which the summary names
+                ops.gemm(x, r, K, N, G, counters=cnt, out=out)
         torch.cuda.synchronize()
         del r, x, out
     for _, M, K, N in SQ_DENSE:  # the vendor library's dense GEMM on fp16 weights of the same shape
@@ -978,7 +992,7 @@ def rocprof_summary(trace_dir: str, command: str, section: str) -> str:
             "",
         ]
         for kern in DECODE_KERNELS:
-            pairs = [(M, N, K) for M in M_SET for _, K, N in LAYER if ops.plan_info(M, N, K, G).function == kern]
+            pairs = [(M, N, K) for M in M_SET for _, K, N in LAYER if launched(ops, M, N, K).function == kern]
             ds = [d for (k, *_), v in groups.items() if k.startswith(kern + "<") for d in v]
             if not pairs or not ds:
                 continue
@@ -1118,7 +1132,7 @@ def decode_bench(ops, args, C, linear, step_fn, step_bytes, prober):
             us = median(replay_samples([g], MEDIAN_SAMPLES)) * 1e3 / C
             del g
             b = gemm_bytes(M, N, K)
-            info = ops.plan_info(M, N, K, G)
+            info = launched(ops, M, N, K)
             probe = prober.us(b, info.workgroups, info.threads)
             best_us, best_g, best_b = prober.best(b)
             kern = info.function
@@ -1208,7 +1222,7 @@ def linears_bench(ops, dev, prober, shapes, Ms, dtype=torch.float16, copies: int
                 it = iter(range(10 ** 9))
                 us = median(call_samples(lambda: call(next(it) % copies), MEDIAN_SAMPLES)) * 1e3
             b, fl = gemm_bytes(M, N, K), 2 * M * N * K
-            info = ops.plan_info(M, N, K, G)
+            info = launched(ops, M, N, K)
             e = {"us": round(us, 2), "GB/s": round(b / us / 1e3, 1), "TFLOP/s": round(fl / us / 1e6, 1),
                  "kernel": info.function, "grid": info.workgroups, "k_slices": info.k_slices}
             e.update({"frac_hbm": round(b / us / 1e3 / HBM_PEAK_GBS, 4),
@@ -1344,7 +1358,7 @@ def planner_sweep(ops, dev, groups, Ms) -> None:
                         ops.clear_plan_overrides()
                         for k, v in (ov or {}).items():
                             ops.set_plan_override(k, v)
-                        i = ops.plan_info(M, N, K, G)
+                        i = launched(ops, M, N, K)
                         key = f"{i.function} {i.variant} ks{i.k_slices} {i.workgroups}x{i.threads}"
                         if ov is None:
                             default = key

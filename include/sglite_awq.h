@@ -263,7 +263,14 @@ int64_t awq_gated_mlp_take_errors(int32_t* counters, int64_t counter_bytes, awq_
  *                            (default 0: in a second kernel)
  *   AWQ_PLAN_FIXUP_POLLS     how often a k-slice workgroup polls for its
  *                            tile's other slices before it leaves the sum to
- *                            the last one (0: never waits) */
+ *                            the last one (0: never waits)
+ *   AWQ_PLAN_RING            0: 17-64 rows keep the kernel above instead of
+ *                            ring_kernel; otherwise its shape code
+ *                            MT*100000 + NTW*10000 + WN*100 + WK (any other
+ *                            value leaves the plan alone)
+ *   AWQ_PLAN_RING_KS         its k-slices, as far as the plan's workspace
+ *                            holds their partials
+ * Any of the other knobs, while set, also keeps ring_kernel out. */
 enum {
   AWQ_PLAN_GEMV_MAX_M = 0,
   AWQ_PLAN_GEMV_VARIANT = 1,
@@ -275,7 +282,9 @@ enum {
   AWQ_PLAN_TILED_KS = 7,
   AWQ_PLAN_KSLICE_VARIANT = 8,
   AWQ_PLAN_TILED_FIXUP = 9,
-  AWQ_PLAN_FIXUP_POLLS = 10
+  AWQ_PLAN_FIXUP_POLLS = 10,
+  AWQ_PLAN_RING = 11,
+  AWQ_PLAN_RING_KS = 12
 };
 int awq_set_plan_override(int knob, int value);
 void awq_clear_plan_overrides(void);
@@ -303,6 +312,11 @@ int awq_gemm_plan_info(int64_t M, int64_t N, int64_t K, int64_t G, int activatio
 /* 1 if that plan splits K on the tiled kernels and sums the k-slices inside
  * the GEMM kernel (when awq_w4a16_gemm is given counters), 0 otherwise. */
 int awq_gemm_plan_fixup(int64_t M, int64_t N, int64_t K, int64_t G, int activation);
+/* The shape code of ring_kernel (AWQ_PLAN_RING) if the launch takes it in
+ * place of the kernel that awq_gemm_plan_info describes (17-64 rows), and its
+ * k-slices in *k_slices; 0 if not.  It needs no counters and no more workspace
+ * than the plan reports. */
+int awq_gemm_plan_ring(int64_t M, int64_t N, int64_t K, int64_t G, int activation, int* k_slices);
 int awq_stream_probe(const void* src, int64_t bytes, int64_t grid, int block, uint32_t* sink, int64_t sink_bytes,
                      awq_stream_t stream);
 /* awq_mfma_probe: `grid` workgroups of `block` threads (64..256), each wave

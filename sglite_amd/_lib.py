@@ -61,6 +61,7 @@ SIGNATURES = {
     "awq_device_cu_count": (_int, []),
     "awq_gemm_plan_info": (_int, [_i64, _i64, _i64, _i64, _int, ctypes.POINTER(_i64)]),
     "awq_gemm_plan_fixup": (_int, [_i64, _i64, _i64, _i64, _int]),
+    "awq_gemm_plan_ring": (_int, [_i64, _i64, _i64, _i64, _int, ctypes.POINTER(_int)]),
     "awq_stream_probe": (_int, [_vp, _i64, _i64, _int, _vp, _i64, _vp]),
     "awq_mfma_probe": (_int, [_i64, _i64, _int, _vp, _i64, _vp]),
     "awq_moe_expert_strides": (_int, [_i64, _i64, _i64, ctypes.POINTER(_i64), ctypes.POINTER(_i64),
@@ -89,6 +90,8 @@ AWQ_PLAN_TILED_KS = 7
 AWQ_PLAN_KSLICE_VARIANT = 8
 AWQ_PLAN_TILED_FIXUP = 9
 AWQ_PLAN_FIXUP_POLLS = 10
+AWQ_PLAN_RING = 11
+AWQ_PLAN_RING_KS = 12
 
 # The header revision this binding follows (AWQ_ABI_VERSION).
 AWQ_ABI_VERSION = 4

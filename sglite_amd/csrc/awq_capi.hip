@@ -549,6 +549,21 @@ int awq_gemm_plan_fixup(int64_t M, int64_t N, int64_t K, int64_t G, int activati
   return p.kind == 1 && p.ks > 1 && p.fixup ? 1 : 0;
 }
 
+int awq_gemm_plan_ring(int64_t M, int64_t N, int64_t K, int64_t G, int activation, int* k_slices) {
+  int64_t Gr = 0;
+  const int st = check_shape(K, N, G, AWQ_DTYPE_FP16, &Gr);
+  if (st != 0) return st;
+  if (M <= 0) return fail(AWQ_STATUS_INVALID_ARGUMENT, "awq_gemm_plan_ring: M must be positive");
+  if (activation != 0 && activation != AWQ_ACT_SILU && activation != AWQ_ACT_GELU)
+    return fail(AWQ_STATUS_INVALID_ARGUMENT, "awq_gemm_plan_ring: unknown activation %d", activation);
+  if (activation != 0 && N % 32 != 0)
+    return fail(AWQ_STATUS_INVALID_ARGUMENT, "a gate/up projection needs N %% 32 == 0, got %lld", (long long)N);
+  if (!k_slices) return fail(AWQ_STATUS_INVALID_ARGUMENT, "awq_gemm_plan_ring: null pointer argument");
+  const GemmPlan p = plan_gemm(make_geom(M, N, K, Gr), activation == 0 ? kActNone : kActSilu);
+  *k_slices = p.ring_ks;
+  return p.ring;
+}
+
 int awq_mfma_probe(int64_t iters, int64_t grid, int block, float* sink, int64_t sink_bytes, awq_stream_t stream) {
   if (iters < 1 || iters >= (int64_t(1) << 40))
     return fail(AWQ_STATUS_INVALID_ARGUMENT, "awq_mfma_probe: iters must be in [1, 2^40)");

@@ -38,8 +38,8 @@ namespace {
 // Planner overrides (tests and sweeps only; see awq_set_plan_override).  An
 // unset knob holds kUnset and the planner's own choice stands.
 constexpr int kUnset = INT_MIN;
-std::atomic<int> g_override[kPlanKnobs] = {kUnset, kUnset, kUnset, kUnset, kUnset, kUnset,
-                                           kUnset, kUnset, kUnset, kUnset, kUnset};
+std::atomic<int> g_override[kPlanKnobs] = {kUnset, kUnset, kUnset, kUnset, kUnset, kUnset, kUnset,
+                                           kUnset, kUnset, kUnset, kUnset, kUnset, kUnset};
 
 int knob(int k, int dflt) {
   const int v = g_override[k].load(std::memory_order_relaxed);
@@ -335,7 +335,86 @@ bool plan_kslice(const Geom& g, int v, int act, GemmPlan& p) {
 // 16-slice 32-row tiled kernel; o_proj 4096 x 2560 at M = 32: 12.32 against
 // 11.59).
 
+// ring_kernel (awq_ring.hip) in place of the tiled plan p at 17-64 rows.
+// (The GEMV and decode kernels' plans stay: those scale each group's sum in
+// fp32, where this kernel, like the tiled ones, rounds every weight.)
+//
+// Column tiles per workgroup (t) and k-slices (ks) come from a cost model
+// fitted to sweeps of every shape over the Qwen3-4B, Llama-3-8B and
+// tensor-parallel linears at M = 20 .. 64: us = a launch + k-tiles of a
+// workgroup x the time of one (more tiles cost dequantisation and MFMAs, more
+// rows activation traffic) + the partials' second kernel; a workgroup's ring
+// fills most of a CU's LDS, so the grid is at most one per CU.  Larger layers
+// (70B-sized qkv, gate_up and down, 1.1-1.3 times slower here) keep the tiled
+// plan, and so do more than 32 k-tiles a slice, the 64-row form with four
+// groups per k-tile (spills; 4096 x 2560 of G = 32 and deeper 1.1-1.6 times
+// slower) and its deep K with two (0.95-0.98).
+// Graph-replay A/B at M = 17-64 over 300 cases: 1.2 times faster on average
+// (Qwen3-4B qkv / o / gate_up / down at M = 32 fp16 11.4 -> 7.7 / 11.1 -> 7.9 /
+// 16.4 -> 12.7 / 12.5 -> 11.4 us; Llama-3-8B qkv / o / gate_up / down at
+// M = 64 14.9 -> 12.8 / 13.8 -> 11.4 / 33.1 -> 25.2 / 20.1 -> 19.8).
+void plan_ring(const Geom& g, int act, GemmPlan& p) {
+  const int forced = knob(kPlanRing, -1);
+  if (forced == 0 || (p.kind != 1 && forced < 0) || g.M < 17 || g.M > 64) return;
+  // An override of the plan it would replace leaves that plan alone.
+  for (int k = 0; k < kPlanRing; ++k)
+    if (knob(k, kUnset) != kUnset && forced < 0) return;
+  // 32-bit buffer ranges and offsets, past-the-end offsets bit 31.
+  const int64_t lim = int64_t(1) << 31;
+  if (g.NT * g.KT * 1024 >= lim || g.M * g.K * 2 >= lim) return;
+  const int64_t slice = g.M * g.NT * 16 * 4;
+  const int mt = (int)(g.M + 15) / 16;
+  const int gpt = (g.NG > 1 && g.G < 128) ? (int)(128 / g.G) : 1;
+  if (mt == 4 && (gpt == 4 || (gpt == 2 && g.KT >= 64)) && forced < 0) return;
+  double best = 0.0;
+  for (int t : {1, 2, 4, 6, 8}) {
+    if (act && t == 1) continue;
+    const int ntw = t <= 2 && !act ? 1 : 2, wn = t / ntw;
+    const int64_t cols = act ? (g.NT / 2 + t / 2 - 1) / (t / 2) : (g.NT + t - 1) / t;
+    const double per_kt = t == 1          ? 0.06 + 0.0475 * mt
+                          : t == 2 && act ? 0.15 * mt - 0.07
+                          : t == 2        ? 0.11 + 0.045 * mt
+                          : t == 4        ? 0.16 + 0.065 * mt
+                          : t == 6        ? 0.28 + 0.085 * mt
+                                          : 0.28 + 0.095 * mt;
+    for (int ks : {1, 2, 3, 4, 6, 8}) {
+      if (ks > 1 && (t > 4 || ks * slice > p.ws_bytes || ks > g.KT / 4)) break;
+      const int64_t ktc = (g.KT + ks - 1) / ks, kse = (g.KT + ktc - 1) / ktc;
+      if (cols * kse > g.cus || ktc > (kse > 1 && mt == 2 ? 31 : 32)) continue;
+      double us = 3.2 + 0.2 * mt + (double)ktc * per_kt;
+      if (kse > 1) us += 1.2 + 0.2 * mt + (double)(kse * slice) * 0.6e-6;
+      if (best == 0.0 || us < best) {
+        best = us;
+        // Eight k-waves where one or two tiles leave room for them and K is
+        // unsplit (4096 x 6144 at M = 32: 10.1 -> 9.6 us).
+        const int wk = mt == 2 && t <= 2 && !act && kse == 1 && g.KT >= (t == 1 ? 16 : 32) ? 8 : 4;
+        p.ring = mt * 100000 + ntw * 10000 + wn * 100 + wk;
+        p.ring_ks = (int)kse;
+        p.ring_ktc = (int)ktc;
+      }
+    }
+  }
+  if (forced > 0 && forced / 100000 == mt && ring_variant_ok(forced, act)) {
+    const int64_t fks = std::min<int64_t>(std::max(knob(kPlanRingKs, 1), 1), 16);
+    p.ring = forced;
+    p.ring_ktc = (int)((g.KT + fks - 1) / fks);
+    p.ring_ks = (int)((g.KT + p.ring_ktc - 1) / p.ring_ktc);
+    if (p.ring_ks > 1 && p.ring_ks * slice > p.ws_bytes) {
+      p.ring_ks = 1;
+      p.ring_ktc = (int)g.KT;
+    }
+  }
+}
+
+GemmPlan plan_kernels(const Geom& g, int act);
+
 GemmPlan plan_gemm(const Geom& g, int act) {
+  GemmPlan p = plan_kernels(g, act);
+  plan_ring(g, act, p);
+  return p;
+}
+
+GemmPlan plan_kernels(const Geom& g, int act) {
   GemmPlan p{};
   const int ksv = knob(kPlanKsliceVariant, 0);
   if (ksv != 0 && plan_kslice(g, ksv, act, p)) return p;
@@ -611,6 +690,7 @@ int plan_threads(const GemmPlan& p) {
 hipError_t launch_gemm(const GemmPlan& p, const void* x, const void* w, const void* sr, const void* zr,
                        const void* bias, void* out, int dtype, const Geom& g, void* ws, int32_t* counters,
                        int64_t counter_bytes, int act, hipStream_t s) {
+  if (p.ring != 0) return launch_ring(p, x, w, sr, zr, bias, out, dtype, g, ws, act, s);
   // The decode kernels' per-column-tile counters follow the split tiles' ones.
   int32_t* col = counters != nullptr && counter_bytes >= kFixupBytes ? counters + kFixupBytes / 4 : nullptr;
   if (p.kind == 0) return launch_skinny(p, x, w, sr, zr, bias, out, dtype, g, ws, col, act, s);

@@ -31,7 +31,9 @@ enum : int {
   kPlanKsliceVariant = 8, // in-kernel split-K decode kernel shape wn*100 + wk*10 + kpw
   kPlanTiledFixup = 9,    // 0: tiled split-K plans sum their slices in a second kernel
   kPlanFixupPolls = 10,   // poll bound of the in-kernel split-K reduction (0: only the last arrival reduces)
-  kPlanKnobs = 11
+  kPlanRing = 11,         // 0: never ring_kernel; otherwise its shape code
+  kPlanRingKs = 12,       // ring_kernel k-slices
+  kPlanKnobs = 13
 };
 bool set_plan_override(int knob, int value);
 void clear_plan_overrides();
@@ -58,6 +60,10 @@ struct GemmPlan {
   int64_t lds_bytes;  // dynamic LDS (GEMV)
   int fixup;          // tiled split K: the k-slice workgroups sum the slices (awq_fixup.h)
   int polls;          // ... each polling at most this often for the tile's other slices
+  int ring;           // shape code of ring_kernel where the launch takes it in place of the kernel above
+                      // (MT * 100000 + NTW * 10000 + WN * 100 + WK), else 0
+  int ring_ks;        // ... its k-slices (their partials within ws_bytes)
+  int ring_ktc;       // ... and k-tiles per slice
 };
 
 // act: fused gate/up activation of the output (0 none, 1 silu, 2 gelu; the
@@ -78,6 +84,11 @@ int64_t tiled_max_k(int bm);
 hipError_t launch_tiled(const GemmPlan& p, const void* x, const void* w, const void* sr, const void* zr,
                         const void* bias, void* out, int dtype, const Geom& g, void* ws, int32_t* counters, int act,
                         hipStream_t s);
+bool ring_variant_ok(int code, int act);
+hipError_t launch_splitk_reduce(const float* part, const void* bias, void* out, const Geom& g, int ks, int act,
+                                int dtype, hipStream_t s);
+hipError_t launch_ring(const GemmPlan& p, const void* x, const void* w, const void* sr, const void* zr,
+                       const void* bias, void* out, int dtype, const Geom& g, void* ws, int act, hipStream_t s);
 // `counters`: the caller's counters buffer (awq_counter_bytes: the split
 // tiles' counters of the tiled kernels, then one int32 per column tile for
 // the decode kernels) of `counter_bytes` bytes, or null.

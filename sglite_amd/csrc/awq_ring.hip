@@ -1,0 +1,293 @@
+// W4A16 GEMM for 17-64 rows on wide layers: many waves per workgroup, the
+// activations through a ring of k-steps in LDS.
+//
+// A workgroup owns 2 * WN column tiles (with a gated activation WN gate tiles
+// and their up tiles) and all M rows; WN * WK waves.  Wave (wn, kw) owns two of
+// the tiles and every WK-th k-tile, so a step is WK k-tiles and the WN waves of
+// a k-tile share its activations.  Every wave has the weights, zero points and
+// scales of its next L k-tiles in flight in registers, and the step's
+// activations arrive L steps ahead by LDS-DMA in a ring of L + 1 slots.  The
+// WK partial sums meet in LDS at the end.
+//
+// What bounds these shapes is not the weight stream but the dequantisation,
+// LDS reads and MFMAs of a k-tile following one another in one or two waves of
+// a SIMD; here a CU runs 8 to 16 waves on one column group.
+#include <algorithm>
+
+#include "awq_buffer.h"
+#include "awq_epilogue.h"
+#include "awq_launch.h"
+
+namespace sgl_awq {
+
+namespace {
+
+constexpr int kRingLds = 160 * 1024;
+constexpr uint32_t kPastEnd = 0x80000000u;  // past every buffer range (below 2^31): such a load returns zeros
+
+struct RingArgs {
+  const void* x;
+  const void* w;
+  const void* s;
+  const void* z;
+  const void* bias;
+  void* out;
+  float* part;
+  int M, N, K, NT, KT, NG, gshift;
+  int ktc, ks;  // k-tiles per slice, slices
+  int WN, WK, act;
+};
+
+// x slots: [k-tile of the step][row][16 chunks of 16 bytes], chunk q of row r
+// at position q ^ (r & 15): a DMA instruction brings four rows of 256
+// contiguous bytes, and the 16 rows that a fragment read touches at one chunk
+// lie in 16 different positions.
+template <int MT, int NTW, int NX, int GPT, typename DT>
+__global__ __launch_bounds__(1024, 4) void ring_kernel(RingArgs a) {
+  using E = typename DT::elem;
+  using V8 = typename DT::vec8;
+  constexpr int BPG = 4 / GPT;
+  constexpr int XT = MT * 256;  // 16-byte vectors of one k-tile's activations
+  extern __shared__ u32x4 ring[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int WN = a.WN, WK = a.WK;
+  const int wn = wave % WN, kw = wave / WN;
+  const int c = lane & 15, lg = lane >> 4;
+  const bool paired = a.act != kActNone;
+  const int half = a.NT >> 1;
+  constexpr int HT = NTW > 1 ? NTW / 2 : 1;  // gate tiles of a wave with a gated activation
+  uint32_t tile[NTW], past[NTW];
+#pragma unroll
+  for (int j = 0; j < NTW; ++j) {
+    const int t = paired ? (blockIdx.x * WN + wn) * HT + j % HT + j / HT * half : (blockIdx.x * WN + wn) * NTW + j;
+    const bool in = t < (paired ? half + j / HT * half : a.NT);
+    tile[j] = in ? (uint32_t)t : 0u;
+    past[j] = in ? 0u : kPastEnd;
+  }
+  const int kt_begin = blockIdx.y * a.ktc, kt_end = min(kt_begin + a.ktc, a.KT);
+  const int steps = (kt_end - kt_begin + WK - 1) / WK;
+  const DqK dk = dq_consts();
+
+  const __amdgpu_buffer_rsrc_t xr = make_rsrc(a.x, (uint32_t)a.M * (uint32_t)a.K * 2u);
+  const __amdgpu_buffer_rsrc_t wr = make_rsrc(a.w, (uint32_t)a.NT * (uint32_t)a.KT * 1024u);
+  const __amdgpu_buffer_rsrc_t zr = make_rsrc(a.z, (uint32_t)a.NT * (uint32_t)a.NG * 8u);
+  const __amdgpu_buffer_rsrc_t sr = make_rsrc(a.s, (uint32_t)a.NT * (uint32_t)a.NG * 32u);
+
+  // The wave's share of its k-tile's activations: NX groups of four rows (a
+  // group past the last repeats it, so that every wave counts NX loads).
+  uint32_t xoff[NX];
+  int xdst[NX], xk[NX];
+#pragma unroll
+  for (int i = 0; i < NX; ++i) {
+    const int rg = min(wn + i * WN, MT * 4 - 1);
+    const int row = rg * 4 + (lane >> 4);
+    const int q = (lane & 15) ^ (row & 15);
+    xoff[i] = row < a.M ? ((uint32_t)row * (uint32_t)a.K + (uint32_t)q * 8u) * 2u : kPastEnd;
+    xk[i] = q * 8;
+    xdst[i] = rg * 64;
+  }
+
+  struct Stage {
+    u32x4 q[NTW];
+    uint32_t z[NTW][GPT];
+    uint16_t s[NTW][GPT];
+  };
+  // Step i's loads in the order the wait counts rely on: activations, weights.
+  auto issue = [&](Stage& st, int i, int slot) {
+    const int kt = kt_begin + i * WK + kw;
+    const uint32_t dead = kt < kt_end ? 0u : kPastEnd;
+    u32x4* dst = ring + (slot * WK + kw) * XT;
+#pragma unroll
+    for (int n = 0; n < NX; ++n) {
+      const uint32_t off = kt * 128 + xk[n] < a.K ? xoff[n] | dead : kPastEnd;
+      load_lds16(xr, dst + xdst[n], off, kt * 256);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < NTW; ++j)
+      st.q[j] = __builtin_amdgcn_raw_buffer_load_b128(wr, (uint32_t)lane * 16u | dead | past[j],
+                                                      (tile[j] * a.KT + kt) * 1024, kCacheStream);
+#pragma unroll
+    for (int gg = 0; gg < GPT; ++gg) {
+      const int g = min((kt * 128 + 32 * BPG * gg) >> a.gshift, a.NG - 1);
+#pragma unroll
+      for (int j = 0; j < NTW; ++j) {
+        st.z[j][gg] = __builtin_amdgcn_raw_buffer_load_b32(zr, (uint32_t)(c >> 3) * 4u | dead | past[j],
+                                                           (tile[j] * a.NG + g) * 8, 0);
+        st.s[j][gg] = __builtin_amdgcn_raw_buffer_load_b16(sr, (uint32_t)c * 2u | dead | past[j],
+                                                           (tile[j] * a.NG + g) * 32, 0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  f32x4 acc[MT][NTW];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int j = 0; j < NTW; ++j) acc[mt][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  auto mul = [&](const Stage& st, const u32x4* xs) {
+    typename Dq<DT>::ZS zs[NTW][GPT];
+#pragma unroll
+    for (int gg = 0; gg < GPT; ++gg)
+#pragma unroll
+      for (int j = 0; j < NTW; ++j) zs[j][gg] = Dq<DT>::make((st.z[j][gg] >> (4 * (c & 7))) & 0xFu, st.s[j][gg]);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      V8 b[MT];
+      const int at = c * 16 + ((w * 4 + lg) ^ c);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) b[mt] = __builtin_bit_cast(V8, xs[mt * 256 + at]);
+#pragma unroll
+      for (int j = 0; j < NTW; ++j) {
+        const V8 v = Dq<DT>::word(st.q[j][w], zs[j][w / BPG], dk);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[mt][j] = mfma16x16x32(v, b[mt], acc[mt][j]);
+      }
+    }
+  };
+
+  // Step i: wait until its loads have landed, meet the other waves at a bare
+  // barrier -- every wave's share of the step is in LDS then, and every wave is
+  // done with step i - 1, whose slot step i + 1 takes -- and issue step i + 1.
+  // The step past the last loads zeros and is never multiplied.  The loop
+  // leaves by a branch past no load, so each stage keeps its registers.  (Four
+  // slots, three steps ahead, leave room for half the waves: slower, see
+  // above.)
+  Stage st[2];
+  issue(st[0], 0, 0);
+  [&] {
+    for (int i = 0;;) {
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        issue(st[1 - d], i + 1, 1 - d);
+        mul(st[d], ring + (d * WK + kw) * XT);
+        if (++i >= steps) return;
+      }
+    }
+  }();
+
+  // The k-waves' partial sums, in the ring's space once its last loads landed
+  // and every wave is done with it.
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+  __syncthreads();
+  f32x4* red = (f32x4*)ring;
+  const int NQ = WN * NTW * MT * 64;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int j = 0; j < NTW; ++j) red[kw * NQ + ((wn * NTW + j) * MT + mt) * 64 + lane] = acc[mt][j];
+  __syncthreads();
+  auto sum = [&](int q) {
+    f32x4 v = red[q];
+    for (int o = 1; o < WK; ++o) v += red[o * NQ + q];
+    return v;
+  };
+  const int64_t Np = (int64_t)a.NT * 16;
+  float* part = a.part + (int64_t)blockIdx.y * a.M * Np;
+  // Quad q: lane l = q % 64 of fragment (wn', j, mt) holds row 16 mt + l % 16
+  // and columns 4 (l / 16) .. + 3.
+  const bool gate = paired && a.ks == 1;
+  const int per = gate ? WN * HT * MT * 64 : NQ;
+  for (int q = threadIdx.x; q < per; q += blockDim.x) {
+    const int l = q & 63, f = q >> 6;
+    const int mt = f % MT, m = mt * 16 + (l & 15), c4 = 4 * (l >> 4);
+    if (m >= a.M) continue;
+    if (gate) {
+      const int w = f / MT / HT, j = f / MT % HT;
+      const int t = (blockIdx.x * WN + w) * HT + j;
+      if (t >= half) continue;
+      const int q0 = ((w * NTW + j) * MT + mt) * 64 + l;
+      store4_act<DT>((E*)a.out, (const E*)a.bias, m, a.N >> 1, t * 16 + c4, a.N >> 1, sum(q0),
+                     sum(q0 + HT * MT * 64), a.act);
+    } else {
+      const int w = f / MT / NTW, j = f / MT % NTW;
+      const int t = paired ? (blockIdx.x * WN + w) * HT + j % HT : (blockIdx.x * WN + w) * NTW + j;
+      if (t >= (paired ? half : a.NT)) continue;
+      const int n0 = (paired ? t + j / HT * half : t) * 16 + c4;
+      const f32x4 v = sum(q);
+      if (a.ks > 1) *(f32x4*)(part + m * Np + n0) = v;
+      else if (n0 < a.N) store4<DT>((E*)a.out, (const E*)a.bias, m, a.N, n0, v);  // N % 16 == 8: half a tile
+    }
+  }
+}
+
+template <int MT, int NTW, int NX, int GPT, typename DT>
+hipError_t launch_form(const RingArgs& a, dim3 grid, hipStream_t s) {
+  const int lds = std::max(2 * a.WK * MT * 4096, a.WK * a.WN * NTW * MT * 1024);
+  hipLaunchKernelGGL((ring_kernel<MT, NTW, NX, GPT, DT>), grid, dim3(64 * a.WN * a.WK), lds, s, a);
+  return hipGetLastError();
+}
+
+template <int MT, int NTW, typename DT>
+hipError_t launch_ring_f(const RingArgs& a, int gpt, dim3 grid, hipStream_t s) {
+  const int nx = (MT * 4 + a.WN - 1) / a.WN;
+#define SGL_RING(NX_)                                                           \
+  if (nx <= NX_) {                                                              \
+    if (gpt == 1) return launch_form<MT, NTW, NX_, 1, DT>(a, grid, s);          \
+    if (gpt == 2) return launch_form<MT, NTW, NX_, 2, DT>(a, grid, s);          \
+    return launch_form<MT, NTW, NX_, 4, DT>(a, grid, s);                        \
+  }
+  SGL_RING(MT)
+  SGL_RING(MT * 2)
+  SGL_RING(MT * 4)
+#undef SGL_RING
+  return hipErrorInvalidValue;
+}
+
+}  // namespace
+
+// Shapes that are instantiated: at most 16 waves, both ring slots within LDS.
+bool ring_variant_ok(int code, int act) {
+  const int mt = code / 100000, ntw = code / 10000 % 10, wn = code / 100 % 10, wk = code % 100;
+  return code > 0 && code % 10000 < 1000 && mt >= 2 && mt <= 4 && (ntw == 2 || (ntw == 1 && !act)) && wn >= 1 && wk >= 1 &&
+         wn * wk <= 16 && 2 * wk * mt * 4096 <= kRingLds;
+}
+
+hipError_t launch_ring(const GemmPlan& p, const void* x, const void* w, const void* sr, const void* zr,
+                       const void* bias, void* out, int dtype, const Geom& g, void* ws, int act, hipStream_t s) {
+  RingArgs a{};
+  a.x = x;
+  a.w = w;
+  a.s = sr;
+  a.z = zr;
+  a.bias = bias;
+  a.out = out;
+  a.part = (float*)ws;
+  a.M = (int)g.M;
+  a.N = (int)g.N;
+  a.K = (int)g.K;
+  a.NT = (int)g.NT;
+  a.KT = (int)g.KT;
+  a.NG = (int)g.NG;
+  a.gshift = g.gshift;
+  a.ktc = p.ring_ktc;
+  a.ks = p.ring_ks;
+  a.WN = p.ring / 100 % 10;
+  a.WK = p.ring % 100;
+  a.act = act;
+  const int mt = p.ring / 100000, ntw = p.ring / 10000 % 10;
+  if (g.M > mt * 16 || !ring_variant_ok(p.ring, act)) return hipErrorInvalidValue;
+  const int gpt = (g.NG > 1 && g.G < 128) ? (int)(128 / g.G) : 1;
+  const int64_t tiles = act ? g.NT / 2 : g.NT, per = (int64_t)a.WN * (act ? ntw / 2 : ntw);
+  const dim3 grid((unsigned)((tiles + per - 1) / per), (unsigned)p.ring_ks);
+  hipError_t e = hipErrorInvalidValue;
+#define SGL_F(MT_, NTW_)                                                                          \
+  if (mt == MT_ && ntw == NTW_)                                                                   \
+    e = dtype == 0 ? launch_ring_f<MT_, NTW_, F16>(a, gpt, grid, s) : launch_ring_f<MT_, NTW_, BF16>(a, gpt, grid, s);
+  SGL_F(2, 1)
+  SGL_F(2, 2)
+  SGL_F(3, 1)
+  SGL_F(3, 2)
+  SGL_F(4, 1)
+  SGL_F(4, 2)
+#undef SGL_F
+  if (e != hipSuccess || p.ring_ks == 1) return e;
+  return launch_splitk_reduce((const float*)ws, bias, out, g, p.ring_ks, act, dtype, s);
+}
+
+}  // namespace sgl_awq

@@ -531,8 +531,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 }
 
 template <typename DT>
-hipError_t launch_splitk_reduce(const float* part, const void* bias, void* out, const Geom& g, int ks, int act,
-                                hipStream_t s) {
+hipError_t launch_reduce_dt(const float* part, const void* bias, void* out, const Geom& g, int ks, int act,
+                            hipStream_t s) {
   using E = typename DT::elem;
   const int64_t quads = g.M * ((act == kActNone ? g.N : g.N / 2) / 4);
   const dim3 grid((unsigned)((quads + 255) / 256)), block(256);
@@ -1075,10 +1075,16 @@ hipError_t launch_tiled(const GemmPlan& p, const void* x, const void* w, const v
   a.polls = p.polls;
   // Groups per 128-row k-tile: 1 for G >= 128 (or one group), else 128 / G.
   const int gpt = (g.NG > 1 && g.G < 128) ? (int)(128 / g.G) : 1;
-  hipError_t e = dtype == 0 ? launch_dt<F16>(p, a, gpt, s) : launch_dt<BF16>(p, a, gpt, s);
+  const hipError_t e = dtype == 0 ? launch_dt<F16>(p, a, gpt, s) : launch_dt<BF16>(p, a, gpt, s);
   if (e != hipSuccess || p.ks == 1 || fixup) return e;
-  return dtype == 0 ? launch_splitk_reduce<F16>((const float*)ws, bias, out, g, p.ks, act, s)
-                    : launch_splitk_reduce<BF16>((const float*)ws, bias, out, g, p.ks, act, s);
+  return launch_splitk_reduce((const float*)ws, bias, out, g, p.ks, act, dtype, s);
+}
+
+// Sum of the k-slices' partials [ks][M][16 NT] (ks <= 16), for every kernel that leaves them.
+hipError_t launch_splitk_reduce(const float* part, const void* bias, void* out, const Geom& g, int ks, int act,
+                                int dtype, hipStream_t s) {
+  return dtype == 0 ? launch_reduce_dt<F16>(part, bias, out, g, ks, act, s)
+                    : launch_reduce_dt<BF16>(part, bias, out, g, ks, act, s);
 }
 
 }  // namespace sgl_awq

@@ -253,6 +253,8 @@ class PlanInfo(NamedTuple):
     workspace_bytes: int
     function: str = ""    # the __global__ function the GEMM launch runs
     fixup: bool = False   # split K summed inside the GEMM kernel (no second launch, given counters)
+    ring: int = 0         # shape code of ring_kernel where the launch takes it in place of ``function`` (17-64 rows)
+    ring_slices: int = 0  # ... and its k-slices
 
 
 def kernel_function(kind: str, variant: int) -> str:
@@ -272,8 +274,11 @@ def plan_info(M: int, N: int, K: int, group_size: int, activation: Optional[str]
     lib = _lib.load()
     _lib.check(lib.awq_gemm_plan_info(M, N, K, G, act, info), "awq_gemm_plan_info")
     fixup = _lib.check(lib.awq_gemm_plan_fixup(M, N, K, G, act), "awq_gemm_plan_fixup") == 1
+    slices = ctypes.c_int()
+    ring = _lib.check(lib.awq_gemm_plan_ring(M, N, K, G, act, ctypes.byref(slices)), "awq_gemm_plan_ring")
     kind = KERNEL_NAMES[int(info[0])]
-    return PlanInfo(kind, *[int(v) for v in info[1:]], function=kernel_function(kind, int(info[1])), fixup=fixup)
+    return PlanInfo(kind, *[int(v) for v in info[1:]], function=kernel_function(kind, int(info[1])), fixup=fixup,
+                    ring=ring, ring_slices=slices.value)
 
 
 PLAN_KNOBS = {"gemv_max_m": _lib.AWQ_PLAN_GEMV_MAX_M, "gemv_variant": _lib.AWQ_PLAN_GEMV_VARIANT,
@@ -281,7 +286,8 @@ PLAN_KNOBS = {"gemv_max_m": _lib.AWQ_PLAN_GEMV_MAX_M, "gemv_variant": _lib.AWQ_P
               "skinny_ks": _lib.AWQ_PLAN_SKINNY_KS, "tiled_min_m": _lib.AWQ_PLAN_TILED_MIN_M,
               "tiled_bm": _lib.AWQ_PLAN_TILED_BM, "tiled_ks": _lib.AWQ_PLAN_TILED_KS,
               "kslice_variant": _lib.AWQ_PLAN_KSLICE_VARIANT, "tiled_fixup": _lib.AWQ_PLAN_TILED_FIXUP,
-              "fixup_polls": _lib.AWQ_PLAN_FIXUP_POLLS}
+              "fixup_polls": _lib.AWQ_PLAN_FIXUP_POLLS, "ring": _lib.AWQ_PLAN_RING,
+              "ring_ks": _lib.AWQ_PLAN_RING_KS}
 
 
 def set_plan_override(knob: str, value: int) -> None:

@@ -40,7 +40,9 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    if device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -68,6 +70,25 @@ def _on_device(device: torch.device) -> Iterator[None]:
     else:
         with torch.cuda.device(device):
             yield
+
+
+def _undispatched(x: torch.Tensor, *others: Optional[torch.Tensor]) -> bool:
+    """True where the dispatcher would only hand these tensors on to the device implementation: plain tensors
+    outside every mode, trace, transform, profiler and gradient.  A call may then run that implementation
+    itself, without the dispatcher's Python layers (one decode linear of 4096 x 2560 called eagerly at M = 1:
+    23.6 us a call through them, 18.7 without)."""
+    if type(x) is not torch.Tensor or x.is_neg() or torch._is_functional_tensor(x):
+        return False
+    grad = torch.is_grad_enabled()
+    if grad and x.requires_grad:
+        return False
+    for t in others:
+        if t is not None and (type(t) is not torch.Tensor or (grad and t.requires_grad)):
+            return False
+    return (torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
+            and torch._C._functorch.peek_interpreter_stack() is None and torch._C._get_tracing_state() is None
+            and torch.autograd.forward_ad._current_level < 0 and not torch._C._autograd._profiler_enabled()
+            and not torch.compiler.is_compiling())
 
 
 def resolve_group_size(group_size: int, K: int) -> int:
@@ -362,22 +383,24 @@ def _gemm_launch(x: torch.Tensor, w: torch.Tensor, s: torch.Tensor, z: torch.Ten
     if M == 0:
         return
     dev = x.device
+    if dev.index is not None and torch._C._cuda_getDevice() != dev.index:
+        with torch.cuda.device(dev):  # the C ABI's planning fills the current device's CUs
+            return _gemm_launch(x, w, s, z, bias, counters, out, K, N, G, act)
     lib = _lib.load()
-    with _on_device(dev):
-        if act == 0:
-            wsb = _lib.check(lib.awq_workspace_bytes(M, N, K, G), "awq_workspace_bytes")
-        else:
-            wsb = _lib.check(lib.awq_workspace_bytes_act(M, N, K, G), "awq_workspace_bytes_act")
-        ws = _workspace(wsb, dev)
-        cb = 0 if counters is None else counters.numel() * 4
-        if act == 0:
-            _lib.check(lib.awq_w4a16_gemm(x.data_ptr(), w.data_ptr(), s.data_ptr(), z.data_ptr(), _ptr(bias),
-                                          out.data_ptr(), M, N, K, G, dtype_code(x.dtype), _ptr(ws), wsb,
-                                          _ptr(counters), cb, _stream(dev)), "awq_w4a16_gemm")
-        else:
-            _lib.check(lib.awq_w4a16_gemm_act(x.data_ptr(), w.data_ptr(), s.data_ptr(), z.data_ptr(), _ptr(bias),
-                                              out.data_ptr(), M, N, K, G, dtype_code(x.dtype), act, _ptr(ws), wsb,
-                                              _ptr(counters), cb, _stream(dev)), "awq_w4a16_gemm_act")
+    if act == 0:
+        wsb = _lib.check(lib.awq_workspace_bytes(M, N, K, G), "awq_workspace_bytes")
+    else:
+        wsb = _lib.check(lib.awq_workspace_bytes_act(M, N, K, G), "awq_workspace_bytes_act")
+    ws = _workspace(wsb, dev)
+    cb = 0 if counters is None else counters.numel() * 4
+    if act == 0:
+        _lib.check(lib.awq_w4a16_gemm(x.data_ptr(), w.data_ptr(), s.data_ptr(), z.data_ptr(), _ptr(bias),
+                                      out.data_ptr(), M, N, K, G, dtype_code(x.dtype), _ptr(ws), wsb,
+                                      _ptr(counters), cb, _stream(dev)), "awq_w4a16_gemm")
+    else:
+        _lib.check(lib.awq_w4a16_gemm_act(x.data_ptr(), w.data_ptr(), s.data_ptr(), z.data_ptr(), _ptr(bias),
+                                          out.data_ptr(), M, N, K, G, dtype_code(x.dtype), act, _ptr(ws), wsb,
+                                          _ptr(counters), cb, _stream(dev)), "awq_w4a16_gemm_act")
 
 
 @torch.library.custom_op(f"{NAMESPACE}::awq_w4a16_gemm", mutates_args=("counters",), device_types="cuda")
@@ -449,7 +472,7 @@ def _check_counters(counters: torch.Tensor, N: int, device: torch.device) -> Non
         raise ValueError(f"counters must be on {device}, got {counters.device}")
     if not counters.is_contiguous():
         raise ValueError("counters must be contiguous")
-    need = _lib.check(_lib.load().awq_counter_bytes(N), "awq_counter_bytes") // 4
+    need = (_lib.AWQ_COUNTER_TILE_BYTES + (N + 15) // 16 * 4) // 4  # awq_counter_bytes
     if counters.numel() < need:
         raise ValueError(f"counters must hold at least {need} int32 (awq_counter_bytes({N}) bytes), "
                          f"got {counters.numel()}")
@@ -494,6 +517,10 @@ def gemm(x: torch.Tensor, r: Repacked, K: int, N: int, group_size: int, bias: Op
     ncols = N if activation is None else N // 2
     if out is not None:
         _check_out(out, (M, ncols), x.dtype, dev)
+    if out is None and _undispatched(x, r.w, r.s, r.z, bias, counters):
+        out = torch.empty((M, ncols), dtype=x.dtype, device=dev)
+        _gemm_launch(x, r.w, r.s, r.z, bias, counters, out, K, N, G, 0 if activation is None else _GATED_ACT[activation])
+        return out
     if activation is None:
         if out is None:
             return torch.ops.sglite_awq.awq_w4a16_gemm(x, r.w, r.s, r.z, bias, counters, K, N, G)

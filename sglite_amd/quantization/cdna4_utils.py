@@ -153,6 +153,8 @@ def apply_awq_linear(weights: Dict[str, Any], x: torch.Tensor, bias: Optional[to
     N = weights["_output_size"]
     G = weights["_group_size"]
     r = ops.Repacked(weights["qweight"], weights["scales"], weights["qzeros"])
+    if x.dim() == 2:
+        return ops.gemm(x, r, K, N, G, bias=bias, counters=weights["workspace"], activation=activation)
     out_shape = x.shape[:-1] + (N if activation is None else N // 2,)
     y = ops.gemm(x.reshape(-1, x.shape[-1]), r, K, N, G, bias=bias, counters=weights["workspace"],
                  activation=activation)

@@ -591,9 +591,9 @@ def committed_traffic(kernel: str):
 
 # The HIP kernels a decode GEMM launch can run (ops.PlanInfo.function); the
 # tiled kind runs tiled_kernel (16x16x32 MFMAs) or mfma32_kernel (32x32x16).
-DECODE_KERNELS = ("skinny_kernel", "gemv_kernel", "tiled_kernel", "mfma32_kernel", "kslice_kernel")
+DECODE_KERNELS = ("skinny_kernel", "gemv_kernel", "tiled_kernel", "mfma32_kernel", "kslice_kernel", "ring_kernel")
 TRACE_KERNELS = ("skinny_kernel", "gemv_kernel", "tiled_kernel", "mfma32_kernel", "splitk_reduce_kernel", "moe_",
-                 "topk_softmax_kernel", "align_kernel", "kslice_kernel", "mlp_kernel")
+                 "topk_softmax_kernel", "align_kernel", "route_kernel", "kslice_kernel", "mlp_kernel", "ring_kernel")
 
 
 def _trace_rows(trace_dir: str):

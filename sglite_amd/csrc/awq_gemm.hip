@@ -1,7 +1,7 @@
 // W4A16 GEMM planning and dispatch for gfx950: out[M, N] = x[M, K] @ W
 // (+ bias), fp32 accumulation, optionally with the gated activation of a
-// merged gate/up projection fused (out[M, N / 2] = act(gate) * up).  Four
-// kernel kinds share the CDNA4 tile layout (awq_device.h):
+// merged gate/up projection fused (out[M, N / 2] = act(gate) * up).  Five
+// kernels share the CDNA4 tile layout (awq_device.h):
 //
 //  * gemv_kernel (awq_gemv.hip): batches of a few rows, HBM-bound;
 //  * skinny_kernel (awq_skinny.hip): decode batches up to 32 rows, HBM-bound
@@ -10,6 +10,8 @@
 //    mfma32_kernel on 32x32x16 ones): prefill (MFMA-bound), mid-size batches
 //    and 5-32 rows on large or deep matrices, split K summed by a second
 //    reduction kernel (or, on request, inside the GEMM kernel);
+//  * ring_kernel (awq_ring.hip): in place of the tiled kind at 17-64 rows, where
+//    its cost model fits (plan_ring);
 //  * kslice_kernel (awq_kslice.hip): decode batches up to 32 rows, split K
 //    reduced by the last workgroup of each column group (planner override
 //    only).

@@ -1,17 +1,26 @@
-// W4A16 GEMM for 17-64 rows on wide layers: many waves per workgroup, the
-// activations through a ring of k-steps in LDS.
+// W4A16 GEMM for 17-64 rows: many waves per workgroup, the activations through
+// a two-slot ring of k-steps in LDS.
 //
-// A workgroup owns 2 * WN column tiles (with a gated activation WN gate tiles
-// and their up tiles) and all M rows; WN * WK waves.  Wave (wn, kw) owns two of
-// the tiles and every WK-th k-tile, so a step is WK k-tiles and the WN waves of
-// a k-tile share its activations.  Every wave has the weights, zero points and
-// scales of its next L k-tiles in flight in registers, and the step's
-// activations arrive L steps ahead by LDS-DMA in a ring of L + 1 slots.  The
-// WK partial sums meet in LDS at the end.
+// A workgroup owns NTW * WN column tiles (with a gated activation half of them
+// gate tiles, the others their up tiles) and all M rows; WN * WK waves.  Wave
+// (wn, kw) owns NTW of the tiles and every WK-th k-tile, so a step is WK
+// k-tiles and the WN waves of a k-tile share its activations.  A step's
+// weights, zero points and scales (registers) and activations (LDS-DMA into
+// the ring) are in flight during the step before it.  The WK partial sums meet
+// in LDS at the end; K is mostly unsplit.
 //
 // What bounds these shapes is not the weight stream but the dequantisation,
-// LDS reads and MFMAs of a k-tile following one another in one or two waves of
-// a SIMD; here a CU runs 8 to 16 waves on one column group.
+// LDS reads and MFMAs of a k-tile following one another: the tiled kernels put
+// four waves on a CU here, one per SIMD, and needed a second kernel for the K
+// slices that filled the chip.  With 8 to 16 waves on a CU the units overlap.
+// Measured against them (graph replay, us; floor at the copy rate of 4.8 TB/s
+// in brackets): Qwen3-4B at M = 32, fp16, qkv 11.4 -> 7.7 (1.7), o 11.1 -> 7.9
+// (1.1), gate_up 16.4 -> 12.7 (5.4), down 12.5 -> 11.4 (2.7); Llama-3-8B at
+// M = 64 qkv 14.9 -> 12.8 (2.7), o 13.8 -> 11.4 (1.8), gate_up 33.1 -> 25.2
+// (12.5), down 20.1 -> 19.8 (6.3).  Tried: four slots, three steps ahead, with
+// half the waves (gate_up at M = 64 27.6); four tiles per wave and half the
+// waves, which halves the LDS reads (26.0); one m-tile at M = 8, where the GEMV
+// and decode kernels stay ahead (qkv 5.9 against 5.7).
 #include <algorithm>
 
 #include "awq_buffer.h"
@@ -152,9 +161,7 @@ __global__ __launch_bounds__(1024, 4) void ring_kernel(RingArgs a) {
   // barrier -- every wave's share of the step is in LDS then, and every wave is
   // done with step i - 1, whose slot step i + 1 takes -- and issue step i + 1.
   // The step past the last loads zeros and is never multiplied.  The loop
-  // leaves by a branch past no load, so each stage keeps its registers.  (Four
-  // slots, three steps ahead, leave room for half the waves: slower, see
-  // above.)
+  // leaves by a branch past no load, so each stage keeps its registers.
   Stage st[2];
   issue(st[0], 0, 0);
   [&] {

@@ -83,7 +83,7 @@ def _undispatched(x: torch.Tensor, *others: Optional[torch.Tensor]) -> bool:
     if grad and x.requires_grad:
         return False
     for t in others:
-        if t is not None and (type(t) is not torch.Tensor or (grad and t.requires_grad)):
+        if t is not None and (type(t) is not torch.Tensor or t.is_neg() or (grad and t.requires_grad)):
             return False
     return (torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
             and torch._C._functorch.peek_interpreter_stack() is None and torch._C._get_tracing_state() is None

@@ -63,3 +63,48 @@ def test_everything_else_meets_the_op():
     with FakeTensorMode() as mode:
         assert not ops._undispatched(mode.from_tensor(x))
     assert not ops._undispatched(torch.nn.Parameter(x))
+
+
+def _layer(bias, K=512, N=256):
+    from sglite_amd.linear import RowParallelLinear
+    from sglite_amd.quantization import get_quantization_config
+
+    method = get_quantization_config("awq").from_config(
+        {"bits": 4, "group_size": 128, "zero_point": True, "quant_method": "awq"}).get_linear_method()
+    t = oracle.make_awq_linear(K, N, 128, seed=3)
+    d = {k: t[k].to(DEV) for k in ("qweight", "qzeros", "scales")}
+    before = torch.get_default_dtype()
+    torch.set_default_dtype(torch.float16)
+    try:
+        layer = RowParallelLinear(K, N, bias, method)
+        layer.load_state_dict({**d, **({"bias": torch.randn(N, generator=torch.Generator().manual_seed(4)).half().to(DEV)}
+                                       if bias else {})})
+    finally:
+        torch.set_default_dtype(before)
+    return layer
+
+
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("M", [1, 20])
+def test_loaded_layer(bias, M, monkeypatch):
+    """A layer holds Parameters: launched directly, to the op's result; modes, a profiler and a compiler meet the op."""
+    from sglite_amd import ops
+
+    layer = _layer(bias)
+    w = layer._weights
+    x = oracle.make_activation(M, 512, seed=5).to(DEV)
+    ref = torch.ops.sglite_awq.awq_w4a16_gemm(x, w["qweight"], w["scales"], w["qzeros"], layer.bias, w["workspace"],
+                                              512, 256, 128)
+    taken = []
+    check = ops._undispatched
+    monkeypatch.setattr(ops, "_undispatched", lambda *t: taken.append(check(*t)) or taken[-1])
+    assert torch.equal(layer.forward(x), ref) and taken == [True]
+    assert torch.equal(layer.forward(x.view(1, M, 512))[0], ref) and taken == [True, True]
+    with _Seen() as seen:
+        assert torch.equal(layer.forward(x), ref)
+    assert any("awq_w4a16_gemm" in n for n in seen.names)
+    monkeypatch.undo()
+    assert torch.equal(torch.compile(lambda v: layer.forward(v) * 2.0, backend="aot_eager")(x), ref * 2.0)
+    if bias:  # a negated view of the bias keeps its sign
+        layer.bias = torch._neg_view(-layer.bias)
+        assert torch.equal(layer.forward(x), ref)

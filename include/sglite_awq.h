@@ -266,10 +266,11 @@ int64_t awq_gated_mlp_take_errors(int32_t* counters, int64_t counter_bytes, awq_
  *                            the last one (0: never waits)
  *   AWQ_PLAN_RING            0: 17-64 rows keep the kernel above instead of
  *                            ring_kernel; otherwise its shape code
- *                            MT*100000 + NTW*10000 + WN*100 + WK (any other
- *                            value leaves the plan alone)
- *   AWQ_PLAN_RING_KS         its k-slices, as far as the plan's workspace
- *                            holds their partials
+ *                            MT*100000 + NTW*10000 + WN*100 + WK, on any plan
+ *                            of those rows (any other value leaves the plan
+ *                            alone)
+ *   AWQ_PLAN_RING_KS         its k-slices with such a code, as far as the
+ *                            plan's workspace holds their partials
  * Any of the other knobs, while set, also keeps ring_kernel out. */
 enum {
   AWQ_PLAN_GEMV_MAX_M = 0,

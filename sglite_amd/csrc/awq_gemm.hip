@@ -356,18 +356,30 @@ bool plan_kslice(const Geom& g, int v, int act, GemmPlan& p) {
 // 16.4 -> 12.7 / 12.5 -> 11.4 us; Llama-3-8B qkv / o / gate_up / down at
 // M = 64 14.9 -> 12.8 / 13.8 -> 11.4 / 33.1 -> 25.2 / 20.1 -> 19.8).
 void plan_ring(const Geom& g, int act, GemmPlan& p) {
-  const int forced = knob(kPlanRing, -1);
-  if (forced == 0 || (p.kind != 1 && forced < 0) || g.M < 17 || g.M > 64) return;
+  const int forced = knob(kPlanRing, kUnset);
+  if (forced == 0 || g.M < 17 || g.M > 64) return;
   // An override of the plan it would replace leaves that plan alone.
   for (int k = 0; k < kPlanRing; ++k)
-    if (knob(k, kUnset) != kUnset && forced < 0) return;
+    if (knob(k, kUnset) != kUnset) return;
   // 32-bit buffer ranges and offsets, past-the-end offsets bit 31.
   const int64_t lim = int64_t(1) << 31;
   if (g.NT * g.KT * 1024 >= lim || g.M * g.K * 2 >= lim) return;
   const int64_t slice = g.M * g.NT * 16 * 4;
   const int mt = (int)(g.M + 15) / 16;
   const int gpt = (g.NG > 1 && g.G < 128) ? (int)(128 / g.G) : 1;
-  if (mt == 4 && (gpt == 4 || (gpt == 2 && g.KT >= 64)) && forced < 0) return;
+  // A shape code of these rows that is instantiated is taken as it is, on any plan; another value counts for nothing.
+  if (forced != kUnset && forced / 100000 == mt && ring_variant_ok(forced, act)) {
+    const int64_t fks = std::min<int64_t>(std::max(knob(kPlanRingKs, 1), 1), 16);
+    p.ring = forced;
+    p.ring_ktc = (int)((g.KT + fks - 1) / fks);
+    p.ring_ks = (int)((g.KT + p.ring_ktc - 1) / p.ring_ktc);
+    if (p.ring_ks > 1 && p.ring_ks * slice > p.ws_bytes) {
+      p.ring_ks = 1;
+      p.ring_ktc = (int)g.KT;
+    }
+    return;
+  }
+  if (p.kind != 1 || (mt == 4 && (gpt == 4 || (gpt == 2 && g.KT >= 64)))) return;
   double best = 0.0;
   for (int t : {1, 2, 4, 6, 8}) {
     if (act && t == 1) continue;
@@ -394,16 +406,6 @@ void plan_ring(const Geom& g, int act, GemmPlan& p) {
         p.ring_ks = (int)kse;
         p.ring_ktc = (int)ktc;
       }
-    }
-  }
-  if (forced > 0 && forced / 100000 == mt && ring_variant_ok(forced, act)) {
-    const int64_t fks = std::min<int64_t>(std::max(knob(kPlanRingKs, 1), 1), 16);
-    p.ring = forced;
-    p.ring_ktc = (int)((g.KT + fks - 1) / fks);
-    p.ring_ks = (int)((g.KT + p.ring_ktc - 1) / p.ring_ktc);
-    if (p.ring_ks > 1 && p.ring_ks * slice > p.ws_bytes) {
-      p.ring_ks = 1;
-      p.ring_ktc = (int)g.KT;
     }
   }
 }

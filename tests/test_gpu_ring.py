@@ -54,13 +54,13 @@ def _check(M, K, N, G, dtype, act=None, bias=False, seed=0):
 
 
 @pytest.mark.parametrize("M", [17, 32, 33, 48, 49, 64])
-@pytest.mark.parametrize("tiles", [10104, 10108, 10204, 20104, 20204, 20304, 20404, 10302])
+@pytest.mark.parametrize("tiles", [10104, 10108, 10204, 10208, 20104, 20204, 20304, 20404, 10302])
 @pytest.mark.parametrize("G,K,N", [(128, 128, 1032), (64, 1088, 1064), (32, 1184, 1048), (-1, 640, 1040)])
 def test_every_shape(M, tiles, G, K, N):
     """K of one k-tile, of 8.5 and 9.25, of 5; N of an odd number of tiles and half a tile."""
     ops = _ops()
     code = (M + 15) // 16 * 100000 + tiles
-    if 2 * (code % 100) * (M + 15) // 16 * 4096 > 160 * 1024:
+    if 2 * (code % 100) * ((M + 15) // 16) * 4096 > 160 * 1024:
         pytest.skip("the ring does not fit LDS")
     ops.set_plan_override("ring", code)
     info = ops.plan_info(M, N, K, G)
@@ -81,20 +81,38 @@ def test_gated_activation(M, dtype, tiles, act, G):
     _check(M, 640, 2080, G, dtype, act=act, bias=tiles == 20304)
 
 
-PLANNED = [  # (M, K, N, G, act): shapes whose plan takes ring_kernel, with and without split K
-    (32, 2560, 6144, 128, None), (40, 2560, 6144, 64, None), (64, 4096, 2560, 128, None), (33, 4096, 264, 32, None),
-    (32, 9728, 2560, 128, None), (64, 3584, 4096, 128, None), (20, 2560, 9728, 128, "silu"), (64, 4096, 3584, 128, "gelu"),
-    (56, 1024, 4096, 128, None),
+PLANNED = [  # (M, K, N, G, act, shape code, k-slices): every column-tile count the planner uses, unsplit and split
+    (32, 2560, 6144, 128, None, 210204, 1), (17, 4096, 6144, 128, None, 210208, 1), (32, 4096, 6144, 128, None, 210208, 1),
+    (32, 4096, 4096, 128, None, 210108, 1), (40, 2560, 6144, 64, None, 310204, 1), (64, 4096, 2560, 128, None, 410204, 3),
+    (33, 4096, 264, 32, None, 310104, 8), (32, 9728, 2560, 128, None, 220204, 6), (64, 3584, 4096, 128, None, 410104, 1),
+    (56, 1024, 4096, 128, None, 410104, 1), (25, 2560, 19456, 128, "silu", 220304, 1),
+    (48, 2560, 19456, 64, "gelu", 320304, 1), (32, 4096, 28672, 32, "silu", 220404, 1),
+    (64, 4096, 3584, 128, "gelu", 420204, 4),
 ]
 
 
-@pytest.mark.parametrize("M,K,N,G,act", PLANNED)
+@pytest.mark.parametrize("M,K,N,G,act,code,slices", PLANNED)
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_planned_shapes(M, K, N, G, act, dtype):
+def test_planned_shapes(M, K, N, G, act, code, slices, dtype):
     ops = _ops()
-    info = ops.plan_info(M, N, K, G, act)
-    if ops.device_cu_count() == 256 and not (M == 20 and info.kernel != "tiled_kernel"):
-        assert info.ring, info
+    if ops.device_cu_count() == 256:
+        info = ops.plan_info(M, N, K, G, act)
+        assert (info.ring, info.ring_slices) == (code, slices), info
     _check(M, K, N, G, dtype, act=act)
     with ops.plan_overrides(ring=0):
         assert ops.plan_info(M, N, K, G, act).ring == 0
+
+
+@pytest.mark.parametrize("M,K,N,G,act,ks,slices", [
+    (33, 4096, 264, 32, None, 3, 3),       # 11, 11 and 10 k-tiles
+    (64, 4096, 544, 64, "silu", 5, 5),     # 7, 7, 7, 7 and 4; 17 gate/up pairs
+    (20, 9728, 1048, 128, None, 16, 16),   # 5 k-tiles a slice, the last of one
+    (64, 1280, 2080, 128, "silu", 8, 1),   # the plan's workspace holds two slices: unsplit
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_forced_slices(M, K, N, G, act, ks, slices, dtype):
+    ops = _ops()
+    ops.set_plan_override("ring", (M + 15) // 16 * 100000 + 20204)
+    ops.set_plan_override("ring_ks", ks)
+    assert ops.plan_info(M, N, K, G, act).ring_slices == slices
+    _check(M, K, N, G, dtype, act=act, bias=True)

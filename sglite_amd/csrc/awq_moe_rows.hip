@@ -36,47 +36,56 @@ struct RowsArgs {
   int mul_rw;
 };
 
-// The 16-row block `b` of the experts' buckets, counted over the experts in
-// order: its expert and first sorted row (e = -1 past the last block).  One
-// lane per 2 or 8 experts (EPL); every wave of a workgroup finds it by itself.
+// The 16-row blocks of the experts' buckets, counted over the experts in
+// order.  One lane per EPL (2 or 8) experts; every wave of a workgroup finds
+// its blocks by itself.
 template <int EPL>
-__device__ __forceinline__ void find_block(const RowsArgs& a, int b, int lane, int& e, int& rb) {
-  int o[EPL + 1];
+struct Blocks {
+  int r0[EPL], nb[EPL];  // first sorted row and blocks of the lane's experts
+  int excl, incl;        // blocks before the lane's first expert and past its last one
+
+  __device__ __forceinline__ void scan(const RowsArgs& a, int lane) {
+    int o[EPL + 1];
 #pragma unroll
-  for (int i = 0; i <= EPL; ++i) o[i] = a.offsets[min(lane * EPL + i, a.E)];
-  int r0[EPL], nb[EPL], sum = 0;
+    for (int i = 0; i <= EPL; ++i) o[i] = a.offsets[min(lane * EPL + i, a.E)];
+    int sum = 0;
 #pragma unroll
-  for (int i = 0; i < EPL; ++i) {
-    r0[i] = min(max(o[i], 0), a.sorted_cap);
-    const int r1 = min(max(o[i + 1], r0[i]), a.sorted_cap);
-    nb[i] = lane * EPL + i < a.E ? (r1 - r0[i]) >> 4 : 0;
-    sum += nb[i];
-  }
-  int incl = sum;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int u = __shfl_up(incl, d);
-    if (lane >= d) incl += u;
-  }
-  const int excl = incl - sum;
-  const uint64_t hit = __ballot(b >= excl && b < incl);
-  if (hit == 0) {
-    e = -1;
-    return;
-  }
-  int fe = 0, fr = 0, pos = excl;
-#pragma unroll
-  for (int i = 0; i < EPL; ++i) {
-    if (b >= pos && b < pos + nb[i]) {
-      fe = lane * EPL + i;
-      fr = r0[i] + (b - pos) * 16;
+    for (int i = 0; i < EPL; ++i) {
+      r0[i] = min(max(o[i], 0), a.sorted_cap);
+      const int r1 = min(max(o[i + 1], r0[i]), a.sorted_cap);
+      nb[i] = lane * EPL + i < a.E ? (r1 - r0[i]) >> 4 : 0;
+      sum += nb[i];
     }
-    pos += nb[i];
+    incl = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int u = __shfl_up(incl, d);
+      if (lane >= d) incl += u;
+    }
+    excl = incl - sum;
   }
-  const int src = __builtin_ctzll(hit);
-  e = __builtin_amdgcn_readlane(fe, src);
-  rb = __builtin_amdgcn_readlane(fr, src);
-}
+
+  // Block b's expert and first sorted row; e = -1 past the last block.
+  __device__ __forceinline__ void find(int b, int lane, int& e, int& rb) const {
+    const uint64_t hit = __ballot(b >= excl && b < incl);
+    if (hit == 0) {
+      e = -1;
+      return;
+    }
+    int fe = 0, fr = 0, pos = excl;
+#pragma unroll
+    for (int i = 0; i < EPL; ++i) {
+      if (b >= pos && b < pos + nb[i]) {
+        fe = lane * EPL + i;
+        fr = r0[i] + (b - pos) * 16;
+      }
+      pos += nb[i];
+    }
+    const int src = __builtin_ctzll(hit);
+    e = __builtin_amdgcn_readlane(fe, src);
+    rb = __builtin_amdgcn_readlane(fr, src);
+  }
+};
 
 // Two column tiles per workgroup (with a gate/up activation one gate tile and
 // its up tile), kMaxWaves waves at most, which split K.  What bounds it is the
@@ -105,15 +114,24 @@ __global__ __launch_bounds__(64 * kMaxWaves, GPT < 4 && EPL <= 2 ? 4 : 3) void m
   const int tile0 = blockIdx.x * HT;
   const int kt0 = wave * a.KT / WK, kt1 = (wave + 1) * a.KT / WK;
 
+  // The first block's rows are fetched along with the offsets: blocks of a
+  // table that starts at 0 without gaps start at 16 b.
+  const int c0 = blockIdx.y * 16 + c;
+  const int sid0 = c0 < a.sorted_cap ? a.sorted[c0] : -1;
+  Blocks<EPL> blocks;
+  blocks.scan(a, lane);
   for (int b = blockIdx.y;; b += gridDim.y) {
-    // The block's rows, fetched along with the offsets: blocks of a table
-    // padded to 16 rows start at 16 b.
-    int sid = b * 16 + c < a.sorted_cap ? a.sorted[b * 16 + c] : -1;
     int e, rb;
-    find_block<EPL>(a, b, lane, e, rb);
+    blocks.find(b, lane, e, rb);
     if (e < 0) break;  // the same in every wave
-    if (rb != b * 16) sid = rb + c < a.sorted_cap ? a.sorted[rb + c] : -1;
+    const int sid = rb + c == c0 ? sid0 : a.sorted[rb + c];  // rb + 16 <= sorted_cap
     const bool valid = sid >= 0 && sid < a.num_routed;
+    // Padding alone (a table padded to more than 16 rows): the same in every
+    // wave.  Multiplying it by zeros cost a pass over the weights a block, more
+    // than the pipelined kernel's 64-row passes over it (E = 128, K = 2048, N =
+    // 1536 top-8 silu fp16, tables of 64 rows: T = 8 66.8 -> 37.3 us, 52.9
+    // there; T = 16 94.2 -> 45.5, 53.9; of 256 rows at T = 8 272 -> 88, 193).
+    if (__ballot(valid) == 0) continue;
     const float rw = a.mul_rw && valid ? a.topk_w[sid] : 1.f;
 
     KWave<1, NTW, GPT, DT> kw;
@@ -220,9 +238,8 @@ hipError_t launch_moe_rows(const MoeGemmParams& p, hipStream_t s) {
   const int gpt = (p.g.NG > 1 && p.g.G < 128) ? (int)(128 / p.g.G) : 1;
   const int waves = 2 * p.num_routed > p.E ? 2 : kMaxWaves;
   const int64_t ht = p.epi ? kTiles / 2 : kTiles, cols = p.epi ? p.g.NT / 2 : p.g.NT;
-  // Every non-empty block of a table padded to 16 rows has a routed row.
-  const int64_t blocks = std::min<int64_t>(p.num_routed, p.E + p.num_routed / 16);
-  const dim3 grid((unsigned)((cols + ht - 1) / ht), (unsigned)blocks);
+  // At most one block with rows per routed row; each block of a table padded to 16 rows has one.
+  const dim3 grid((unsigned)((cols + ht - 1) / ht), (unsigned)p.num_routed);
 #define SGL_EPL(N_)                                                               \
   (p.dtype == 0 ? launch_rows<N_, F16>(a, gpt, p.epi, grid, waves, s)             \
                 : launch_rows<N_, BF16>(a, gpt, p.epi, grid, waves, s))

@@ -25,6 +25,8 @@ CASES = [  # (T, E, k, K, N, G, block size, routing)
     (40, 40, 1, 256, 64, 128, 16, "one"),       # all rows on one expert: three blocks, the last of 8 rows
     (24, 26, 1, 256, 64, 128, 64, "two"),       # buckets of 64: blocks of padding alone
     (2, 512, 4, 256, 64, 128, 16, "last"),      # the last expert
+    (1, 4, 1, 256, 64, 128, 1024, "spread"),    # 63 blocks of padding behind one row, one workgroup per column group
+    (5, 130, 7, 256, 64, 128, 256, "spread"),   # padding blocks dealt to every workgroup
 ]
 
 

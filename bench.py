@@ -18,7 +18,7 @@ figure).  Every other duration is also a median of >= 50 samples.
 
 Also reported on the same line:
   roofline      the dominant decode kernel of the step (the one that moves the
-                most of its algorithmic bytes; ops.plan_info names the kernel
+                most of its algorithmic bytes; ops.launch_info names the kernel
                 of each shape): algorithmic
                 bytes of its launches / their durations, measured with HIP events
                 around graphs of back-to-back launches on the launch stream,
@@ -548,7 +548,7 @@ def pmc_summary(fetch_dir: str, write_dir: str) -> str:
     algo = defaultdict(list)
     for M in M_SET:
         for _, K, N in LAYER:
-            algo[launched(ops, M, N, K).function].append(gemm_bytes(M, N, K))
+            algo[ops.launch_info(M, N, K, G).function].append(gemm_bytes(M, N, K))
     lines = [
         "# HBM traffic of the decode kernels (Qwen3-4B layer, M = 1, 8, 32), rocprofv3 PMC",
         "",
@@ -675,21 +675,8 @@ def bounds_bench(ops, dev: torch.device, reps: int = 7) -> dict:
     return out
 
 
-def launched(ops, M: int, N: int, K: int, activation=None):
-    """The plan with the kernel that the launch runs: ring_kernel's grid and k-slices where it takes the place
-    of the planned kernel (17-64 rows)."""
-    info = ops.plan_info(M, N, K, G, activation)
-    if not info.ring:
-        return info
-    ntw, wn, wk = info.ring // 10000 % 10, info.ring // 100 % 10, info.ring % 100
-    tiles = (N + 15) // 16
-    groups = -(-tiles // (wn * ntw)) if activation is None else -(-(tiles // 2) // (wn * ntw // 2))
-    return info._replace(function="ring_kernel", variant=info.ring, k_slices=info.ring_slices,
-                         workgroups=groups * info.ring_slices, threads=64 * wn * wk)
-
-
 def _launches_per_call(ops, M: int, N: int, K: int, activation=None) -> int:
-    info = launched(ops, M, N, K, activation)
+    info = ops.launch_info(M, N, K, G, activation)
     return 2 if info.kernel == "tiled_kernel" and info.k_slices > 1 and not info.fixup else 1
 
 
@@ -992,7 +979,7 @@ def rocprof_summary(trace_dir: str, command: str, section: str) -> str:
             "",
         ]
         for kern in DECODE_KERNELS:
-            pairs = [(M, N, K) for M in M_SET for _, K, N in LAYER if launched(ops, M, N, K).function == kern]
+            pairs = [(M, N, K) for M in M_SET for _, K, N in LAYER if ops.launch_info(M, N, K, G).function == kern]
             ds = [d for (k, *_), v in groups.items() if k.startswith(kern + "<") for d in v]
             if not pairs or not ds:
                 continue
@@ -1132,7 +1119,7 @@ def decode_bench(ops, args, C, linear, step_fn, step_bytes, prober):
             us = median(replay_samples([g], MEDIAN_SAMPLES)) * 1e3 / C
             del g
             b = gemm_bytes(M, N, K)
-            info = launched(ops, M, N, K)
+            info = ops.launch_info(M, N, K, G)
             probe = prober.us(b, info.workgroups, info.threads)
             best_us, best_g, best_b = prober.best(b)
             kern = info.function
@@ -1222,7 +1209,7 @@ def linears_bench(ops, dev, prober, shapes, Ms, dtype=torch.float16, copies: int
                 it = iter(range(10 ** 9))
                 us = median(call_samples(lambda: call(next(it) % copies), MEDIAN_SAMPLES)) * 1e3
             b, fl = gemm_bytes(M, N, K), 2 * M * N * K
-            info = launched(ops, M, N, K)
+            info = ops.launch_info(M, N, K, G)
             e = {"us": round(us, 2), "GB/s": round(b / us / 1e3, 1), "TFLOP/s": round(fl / us / 1e6, 1),
                  "kernel": info.function, "grid": info.workgroups, "k_slices": info.k_slices}
             e.update({"frac_hbm": round(b / us / 1e3 / HBM_PEAK_GBS, 4),
@@ -1358,7 +1345,7 @@ def planner_sweep(ops, dev, groups, Ms) -> None:
                         ops.clear_plan_overrides()
                         for k, v in (ov or {}).items():
                             ops.set_plan_override(k, v)
-                        i = launched(ops, M, N, K)
+                        i = ops.launch_info(M, N, K, G)
                         key = f"{i.function} {i.variant} ks{i.k_slices} {i.workgroups}x{i.threads}"
                         if ov is None:
                             default = key

@@ -61,6 +61,9 @@ const char* awq_version(void);
  *      knobs AWQ_PLAN_TILED_FIXUP / AWQ_PLAN_FIXUP_POLLS are new;
  *   4  the gated MLP block (awq_gated_mlp and its plan, workspace and error
  *      calls) is new.
+ * Calls added since without a change to an existing one keep the revision
+ * (awq_moe_route with AWQ_DTYPE_FP32, awq_gemm_plan_ring, awq_gemm_launch_info,
+ * the AWQ_PLAN_RING knobs): a caller that binds them by name finds out there.
  * No counterpart in the reference (its kernels are Python and Triton). */
 #define AWQ_ABI_VERSION 4
 int awq_abi_version(void);
@@ -133,8 +136,9 @@ int awq_dequant_repacked(const void* w, const void* s, const void* z, int dtype,
  * 16-column tile. */
 #define AWQ_COUNTER_TILE_BYTES (64ll << 10)
 int64_t awq_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t G);
-/* Which kernel awq_w4a16_gemm runs for this shape: 0 = decode split-K kernel,
- * 1 = tiled MFMA kernel, 2 = small-batch GEMV kernel, 3 = k-slice decode
+/* Which kind of plan awq_w4a16_gemm runs for this shape: 0 = decode split-K
+ * kernel, 1 = tiled MFMA kernel (at 17-64 rows mostly ring_kernel in its
+ * place: awq_gemm_launch_info), 2 = small-batch GEMV kernel, 3 = k-slice decode
  * kernel (benchmarks and diagnostics; no counterpart in the reference). */
 int awq_gemm_kernel_kind(int64_t M, int64_t N, int64_t K, int64_t G);
 int64_t awq_counter_bytes(int64_t N);
@@ -296,11 +300,16 @@ void awq_clear_plan_overrides(void);
 int awq_device_cu_count(void);
 
 /* ---- diagnostics and measurement (no counterpart in the reference) ---------
- * awq_gemm_plan_info: the plan that awq_w4a16_gemm (activation 0) or
- * awq_w4a16_gemm_act (AWQ_ACT_SILU / AWQ_ACT_GELU) runs for this shape on the
- * current device, written to info[0..5]: kernel kind (as
- * awq_gemm_kernel_kind), shape code, k-slices across workgroups, workgroups
- * per launch, threads per workgroup, workspace bytes.
+ * awq_gemm_launch_info: what awq_w4a16_gemm (activation 0) or
+ * awq_w4a16_gemm_act (AWQ_ACT_SILU / AWQ_ACT_GELU) launches for this shape on
+ * the current device, written to info[0..5]: kernel kind (as
+ * awq_gemm_kernel_kind, or 4 for ring_kernel), shape code, k-slices across
+ * workgroups, workgroups per launch, threads per workgroup, and the workspace
+ * bytes that the call demands.
+ * awq_gemm_plan_info: the same of the plan that awq_gemm_kernel_kind names and
+ * that sizes the workspace.  The launch is that plan, except at 17-64 rows
+ * where ring_kernel takes the place of a tiled one (awq_gemm_plan_ring): it
+ * runs within the same workspace and leaves the counters alone.
  *
  * awq_stream_probe: streams `bytes` (a multiple of 16, src 16-byte aligned)
  * with `grid` workgroups of `block` threads (64..1024, a multiple of 64),
@@ -310,7 +319,8 @@ int awq_device_cu_count(void);
  * launch of that shape can reach at all (the decode roofline's attainable
  * ceiling). */
 int awq_gemm_plan_info(int64_t M, int64_t N, int64_t K, int64_t G, int activation, int64_t* info);
-/* 1 if that plan splits K on the tiled kernels and sums the k-slices inside
+int awq_gemm_launch_info(int64_t M, int64_t N, int64_t K, int64_t G, int activation, int64_t* info);
+/* 1 if the plan of awq_gemm_plan_info splits K on the tiled kernels and sums the k-slices inside
  * the GEMM kernel (when awq_w4a16_gemm is given counters), 0 otherwise. */
 int awq_gemm_plan_fixup(int64_t M, int64_t N, int64_t K, int64_t G, int activation);
 /* The shape code of ring_kernel (AWQ_PLAN_RING) if the launch takes it in

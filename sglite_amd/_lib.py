@@ -60,6 +60,7 @@ SIGNATURES = {
     "awq_clear_plan_overrides": (None, []),
     "awq_device_cu_count": (_int, []),
     "awq_gemm_plan_info": (_int, [_i64, _i64, _i64, _i64, _int, ctypes.POINTER(_i64)]),
+    "awq_gemm_launch_info": (_int, [_i64, _i64, _i64, _i64, _int, ctypes.POINTER(_i64)]),
     "awq_gemm_plan_fixup": (_int, [_i64, _i64, _i64, _i64, _int]),
     "awq_gemm_plan_ring": (_int, [_i64, _i64, _i64, _i64, _int, ctypes.POINTER(_int)]),
     "awq_stream_probe": (_int, [_vp, _i64, _i64, _int, _vp, _i64, _vp]),

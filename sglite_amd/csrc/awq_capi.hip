@@ -518,23 +518,59 @@ void awq_clear_plan_overrides(void) { clear_plan_overrides(); }
 
 int awq_device_cu_count(void) { return device_cu_count(); }
 
-int awq_gemm_plan_info(int64_t M, int64_t N, int64_t K, int64_t G, int activation, int64_t* info) {
+namespace {
+
+// The plan of awq_gemm_plan_info and awq_gemm_launch_info.
+int query_plan(const char* who, int64_t M, int64_t N, int64_t K, int64_t G, int activation, const int64_t* info,
+               Geom* g, GemmPlan* p) {
   int64_t Gr = 0;
   const int st = check_shape(K, N, G, AWQ_DTYPE_FP16, &Gr);
   if (st != 0) return st;
-  if (M <= 0) return fail(AWQ_STATUS_INVALID_ARGUMENT, "awq_gemm_plan_info: M must be positive");
+  if (M <= 0) return fail(AWQ_STATUS_INVALID_ARGUMENT, "%s: M must be positive", who);
   if (activation != 0 && activation != AWQ_ACT_SILU && activation != AWQ_ACT_GELU)
-    return fail(AWQ_STATUS_INVALID_ARGUMENT, "awq_gemm_plan_info: unknown activation %d", activation);
+    return fail(AWQ_STATUS_INVALID_ARGUMENT, "%s: unknown activation %d", who, activation);
   if (activation != 0 && N % 32 != 0)
     return fail(AWQ_STATUS_INVALID_ARGUMENT, "a gate/up projection needs N %% 32 == 0, got %lld", (long long)N);
-  if (!info) return fail(AWQ_STATUS_INVALID_ARGUMENT, "awq_gemm_plan_info: null pointer argument");
-  const GemmPlan p = plan_gemm(make_geom(M, N, K, Gr), activation == 0 ? kActNone : kActSilu);
+  if (!info) return fail(AWQ_STATUS_INVALID_ARGUMENT, "%s: null pointer argument", who);
+  *g = make_geom(M, N, K, Gr);
+  *p = plan_gemm(*g, activation == 0 ? kActNone : kActSilu);
+  return 0;
+}
+
+void write_plan(const GemmPlan& p, int64_t* info) {
   info[0] = p.kind;
   info[1] = p.variant;
   info[2] = p.ks;
   info[3] = p.grid_x * p.grid_y * (p.kind == 1 || p.kind == 3 ? p.ks : 1);
   info[4] = plan_threads(p);
   info[5] = p.ws_bytes;
+}
+
+}  // namespace
+
+int awq_gemm_plan_info(int64_t M, int64_t N, int64_t K, int64_t G, int activation, int64_t* info) {
+  Geom g;
+  GemmPlan p;
+  const int st = query_plan("awq_gemm_plan_info", M, N, K, G, activation, info, &g, &p);
+  if (st != 0) return st;
+  write_plan(p, info);
+  return ok();
+}
+
+int awq_gemm_launch_info(int64_t M, int64_t N, int64_t K, int64_t G, int activation, int64_t* info) {
+  Geom g;
+  GemmPlan p;
+  const int st = query_plan("awq_gemm_launch_info", M, N, K, G, activation, info, &g, &p);
+  if (st != 0) return st;
+  write_plan(p, info);
+  if (p.ring != 0) {
+    const dim3 grid = ring_grid(p, g, activation == 0 ? kActNone : kActSilu);
+    info[0] = 4;
+    info[1] = p.ring;
+    info[2] = p.ring_ks;
+    info[3] = (int64_t)grid.x * grid.y;
+    info[4] = 64 * (p.ring / 100 % 10) * (p.ring % 100);
+  }
   return ok();
 }
 

@@ -85,6 +85,7 @@ hipError_t launch_tiled(const GemmPlan& p, const void* x, const void* w, const v
                         const void* bias, void* out, int dtype, const Geom& g, void* ws, int32_t* counters, int act,
                         hipStream_t s);
 bool ring_variant_ok(int code, int act);
+dim3 ring_grid(const GemmPlan& p, const Geom& g, int act);
 hipError_t launch_splitk_reduce(const float* part, const void* bias, void* out, const Geom& g, int ks, int act,
                                 int dtype, hipStream_t s);
 hipError_t launch_ring(const GemmPlan& p, const void* x, const void* w, const void* sr, const void* zr,

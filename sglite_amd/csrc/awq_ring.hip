@@ -255,6 +255,13 @@ bool ring_variant_ok(int code, int act) {
          wn * wk <= 16 && 2 * wk * mt * 4096 <= kRingLds;
 }
 
+// Workgroups of a launch: column-tile groups times k-slices.
+dim3 ring_grid(const GemmPlan& p, const Geom& g, int act) {
+  const int ntw = p.ring / 10000 % 10, wn = p.ring / 100 % 10;
+  const int64_t tiles = act ? g.NT / 2 : g.NT, per = (int64_t)wn * (act ? ntw / 2 : ntw);
+  return dim3((unsigned)((tiles + per - 1) / per), (unsigned)p.ring_ks);
+}
+
 hipError_t launch_ring(const GemmPlan& p, const void* x, const void* w, const void* sr, const void* zr,
                        const void* bias, void* out, int dtype, const Geom& g, void* ws, int act, hipStream_t s) {
   RingArgs a{};
@@ -280,8 +287,7 @@ hipError_t launch_ring(const GemmPlan& p, const void* x, const void* w, const vo
   const int mt = p.ring / 100000, ntw = p.ring / 10000 % 10;
   if (g.M > mt * 16 || !ring_variant_ok(p.ring, act)) return hipErrorInvalidValue;
   const int gpt = (g.NG > 1 && g.G < 128) ? (int)(128 / g.G) : 1;
-  const int64_t tiles = act ? g.NT / 2 : g.NT, per = (int64_t)a.WN * (act ? ntw / 2 : ntw);
-  const dim3 grid((unsigned)((tiles + per - 1) / per), (unsigned)p.ring_ks);
+  const dim3 grid = ring_grid(p, g, act);
   hipError_t e = hipErrorInvalidValue;
 #define SGL_F(MT_, NTW_)                                                                          \
   if (mt == MT_ && ntw == NTW_)                                                                   \

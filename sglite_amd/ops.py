@@ -258,8 +258,8 @@ KERNEL_NAMES = {0: "skinny_kernel", 1: "tiled_kernel", 2: "gemv_kernel", 3: "ksl
 
 
 def gemm_kernel(M: int, N: int, K: int, group_size: int, activation: Optional[str] = None) -> str:
-    """Name of the kernel ``gemm`` runs for this shape (with ``activation``:
-    the fused gate/up GEMM's kernel)."""
+    """Name of the kernel kind ``gemm`` plans for this shape (with ``activation``:
+    the fused gate/up GEMM's); ``launch_info`` names the function that runs."""
     G = resolve_group_size(group_size, K)
     lib = _lib.load()
     if activation is None:
@@ -290,7 +290,8 @@ def kernel_function(kind: str, variant: int) -> str:
 
 
 def plan_info(M: int, N: int, K: int, group_size: int, activation: Optional[str] = None) -> PlanInfo:
-    """The plan ``gemm`` runs for this shape on the current device."""
+    """The plan of ``gemm`` for this shape on the current device: what it launches, except where ``ring`` names
+    the form of ring_kernel that runs in its place (``launch_info``)."""
     G = resolve_group_size(group_size, K)
     info = (ctypes.c_int64 * 6)()
     act = 0 if activation is None else _GATED_ACT[activation]
@@ -302,6 +303,19 @@ def plan_info(M: int, N: int, K: int, group_size: int, activation: Optional[str]
     kind = KERNEL_NAMES[int(info[0])]
     return PlanInfo(kind, *[int(v) for v in info[1:]], function=kernel_function(kind, int(info[1])), fixup=fixup,
                     ring=ring, ring_slices=slices.value)
+
+
+def launch_info(M: int, N: int, K: int, group_size: int, activation: Optional[str] = None) -> PlanInfo:
+    """``plan_info`` with the function, shape code, k-slices, workgroups and threads that ``gemm`` launches."""
+    plan = plan_info(M, N, K, group_size, activation)
+    if not plan.ring:
+        return plan
+    info = (ctypes.c_int64 * 6)()
+    act = 0 if activation is None else _GATED_ACT[activation]
+    _lib.check(_lib.load().awq_gemm_launch_info(M, N, K, resolve_group_size(group_size, K), act, info),
+               "awq_gemm_launch_info")
+    return plan._replace(variant=int(info[1]), k_slices=int(info[2]), workgroups=int(info[3]), threads=int(info[4]),
+                         function="ring_kernel")
 
 
 PLAN_KNOBS = {"gemv_max_m": _lib.AWQ_PLAN_GEMV_MAX_M, "gemv_variant": _lib.AWQ_PLAN_GEMV_VARIANT,

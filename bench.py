@@ -956,7 +956,7 @@ def rocprof_summary(trace_dir: str, command: str, section: str) -> str:
 
     decode: the decode step; every (M, linear) is launched equally often, so a
     kernel's mean algorithmic bytes per launch is the mean over the (M, linear)
-    pairs it serves (ops.plan_info names the kernel of each shape); a split-K
+    pairs it serves (ops.launch_info names the kernel of each shape); a split-K
     GEMM on the tiled kernels also runs splitk_reduce_kernel, listed apart.
     prefill-M (--profile-workload prefill-M): the four Llama-3-8B linears at M,
     each launched 2 + PROFILE_REPS times in order; per linear the mean of the

@@ -239,7 +239,9 @@ hipError_t launch_ring_f(const RingArgs& a, int gpt, dim3 grid, hipStream_t s) {
     if (gpt == 2) return launch_form<MT, NTW, NX_, 2, DT>(a, grid, s);          \
     return launch_form<MT, NTW, NX_, 4, DT>(a, grid, s);                        \
   }
-  SGL_RING(MT)
+  if constexpr (NTW > 1) {
+    SGL_RING(MT)
+  }
   SGL_RING(MT * 2)
   SGL_RING(MT * 4)
 #undef SGL_RING
@@ -248,10 +250,12 @@ hipError_t launch_ring_f(const RingArgs& a, int gpt, dim3 grid, hipStream_t s) {
 
 }  // namespace
 
-// Shapes that are instantiated: at most 16 waves, both ring slots within LDS.
+// Shapes that are instantiated: at most 16 waves, both ring slots within LDS;
+// one tile a wave in at most three column waves (the planner takes more than
+// two tiles as two a wave).
 bool ring_variant_ok(int code, int act) {
   const int mt = code / 100000, ntw = code / 10000 % 10, wn = code / 100 % 10, wk = code % 100;
-  return code > 0 && code % 10000 < 1000 && mt >= 2 && mt <= 4 && (ntw == 2 || (ntw == 1 && !act)) && wn >= 1 && wk >= 1 &&
+  return code > 0 && (ntw == 2 || wn <= 3) && code % 10000 < 1000 && mt >= 2 && mt <= 4 && (ntw == 2 || (ntw == 1 && !act)) && wn >= 1 && wk >= 1 &&
          wn * wk <= 16 && 2 * wk * mt * 4096 <= kRingLds;
 }
 

@@ -34,7 +34,8 @@ def test_unusable_codes_leave_the_plan_alone(M, K, N, act, kernel):
     mt = (M + 15) // 16
     for code in (5, -1, 219999, (mt % 3 + 2) * 100000 + 10104,  # no shape; no such waves; another number of m-tiles
                  mt * 100000 + 20909,  # 81 waves
-                 mt * 100000 + 30104):  # three tiles a wave
+                 mt * 100000 + 30104,  # three tiles a wave
+                 mt * 100000 + 10402):  # four column waves of one tile
         ops.set_plan_override("ring", code)
         assert _info(M, K, N, act) == plan, code
     if act:

@@ -16,7 +16,7 @@ linear moves K*N/2 (int4) + (K/128)*N/2 (zeros) + (K/128)*N*2 (scales)
 + 2*M*K (x) + 2*M*N (y) bytes (config.value_from_mean gives the mean-based
 figure).  Every other duration is also a median of >= 50 samples.
 
-Also reported on the same line:
+Printed last, the JSON line also holds:
   roofline      the dominant decode kernel of the step (the one that moves the
                 most of its algorithmic bytes; ops.launch_info names the kernel
                 of each shape): algorithmic
@@ -28,7 +28,12 @@ Also reported on the same line:
                 `attainable_GB/s` / `frac_of_attainable` set it against the
                 streaming probe (awq_stream_probe) run with the same grid, block
                 and bytes: what a launch of that shape reaches with no arithmetic.
-  decode_kernels, per_m   the same per kernel and per batch size, with each
+  cpu_baseline  the CPU oracle on the host cores (dequantisation and matmul timed
+                separately, 2 warm-ups, median of 5) on the Qwen3-4B layer at M = 1,
+                8, 32, in GB/s;
+  summary       the key figures of the sections below.
+The sections come before it, a line "# name: {...}" each:
+  decode_kernels, per_m   these figures per kernel and per batch size, with each
                 linear's probe ceiling (and the best ceiling over a few grids).
   llama3_8b     Llama-3-8B's four linears at M = 1, 16, 256, 2048, 8192
                 (GB/s and fraction of HBM at decode sizes, TFLOP/s and fraction of
@@ -40,9 +45,8 @@ Also reported on the same line:
                 M = 64 (GB/s, one graph per pass) and M = 4096 (TFLOP/s).
   bounds        the MFMA-rate probe (awq_mfma_probe) at one and two waves per
                 SIMD: the compute bound the prefill TFLOP/s are read against.
-  cpu_baseline  the CPU oracle on the host cores for every workload above
-                (dequantisation and matmul timed separately, 2 warm-ups, median
-                of 5); value is the Qwen3-4B layer at M = 1, 8, 32 in GB/s.
+  tp_shards, bf16   tensor-parallel shards; the bf16 kernels.
+  cpu_per_workload  the CPU oracle on every workload above.
 
 Usage: python bench.py [--steps K] [--warmup W] [--gpus 1]
 
@@ -479,7 +483,7 @@ def cpu_baseline(warmup: int = 2, runs: int = 5) -> dict:
     return {"value": round(value, 4), "unit": "GB/s", "cores": threads, "kind": "port",
             "sample": f"CPU oracle (torch dequantise, pinned bit-exact to the numpy oracle, + fp32 matmul + fp16 "
                       f"cast), {warmup} warm-ups then the median of {runs}; value = the Qwen3-4B layer at M = 1, 8, "
-                      f"32; the other workloads in per_workload ({time.perf_counter() - t_start:.1f} s in all); "
+                      f"32; the other workloads in cpu_per_workload ({time.perf_counter() - t_start:.1f} s in all); "
                       f"host {model}, os.cpu_count() = {os.cpu_count()}",
             "per_workload": res}
 
@@ -1359,8 +1363,7 @@ def planner_sweep(ops, dev, groups, Ms) -> None:
 
 
 def headline_summary(dec, prefill, moe, llama, stack, mlp, bounds) -> dict:
-    """The sections' key figures in a few hundred characters, printed last on the JSON line so that a
-    log that keeps only the end of the line still holds them: per decode batch [us per layer, fraction
+    """The sections' key figures in a few hundred characters, last on the JSON line: per decode batch [us per layer, fraction
     of the streaming ceiling, GB/s]; per Llama-3-8B batch [us per layer, fraction of the roofline its
     arithmetic intensity puts it under]; prefill, MoE, 70B-stack, gated-MLP and bound fractions."""
     out: dict = {}
@@ -1555,23 +1558,21 @@ def main() -> int:
                    "value_from_mean": None if dec is None else round(dec["value_mean"], 1),
                    "ms_per_step_mean": None if dec is None else round(dec["ms_per_step_mean"], 5)},
         "roofline": None if dec is None else dec["roofline"],
-        "cpu_baseline": cpu,
-        # The long sections first, the decode summary last: the end of the
-        # line is what a truncated log keeps.
-        "llama3_8b": llama,
-        "tp_shards": tp,
-        "bf16": bf16,
-        "stack70b": stack,
-        "bounds": bounds,
-        "moe": moe,
-        "mlp": mlp,
-        "prefill": prefill,
-        "decode_kernels": None if dec is None else dec["kernels"],
-        "per_m": None if dec is None else dec["per_m"],
+        "cpu_baseline": None if cpu is None else {k: v for k, v in cpu.items() if k != "per_workload"},
         "summary": headline_summary(dec, prefill, moe, llama, stack, mlp, bounds),
     }
-    print(json.dumps(line))
+    sections = {"llama3_8b": llama, "tp_shards": tp, "bf16": bf16, "stack70b": stack, "bounds": bounds, "moe": moe,
+                "mlp": mlp, "prefill": prefill, "decode_kernels": None if dec is None else dec["kernels"],
+                "per_m": None if dec is None else dec["per_m"],
+                "cpu_per_workload": None if cpu is None else cpu["per_workload"]}
+    print("\n".join(report(sections, line)), flush=True)
     return 0
+
+
+def report(sections: dict, line: dict) -> list:
+    """The output: a line "# name: {...}" per section, some of several KB, then the JSON line.  That one stays
+    short, so that a log which keeps the last few KB of the output holds it whole."""
+    return [f"# {name}: {json.dumps(v)}" for name, v in sections.items() if v is not None] + [json.dumps(line)]
 
 
 def progress(what: str) -> None:

@@ -79,3 +79,18 @@ def test_sq_summary_matches_dispatch_order_and_drops_the_warm_up(tmp_path):
         assert cols[5] == "0.20"
         assert cols[7] == "0.30"
         assert cols[-1].split(" / ")[1] == str(5 + i)
+
+
+def test_json_line_is_short_and_last():
+    """A log that keeps 8 KB of the output holds the JSON line: the long sections come before it."""
+    import json
+
+    per_m = {str(m): {"GB/s": 1376.1, "us_per_layer": 1234.567, "frac_of_ceiling": 0.1234, "frac_hbm": 0.1234,
+                      "frac_mfma": 0.1234, "bound": "hbm", "linears": {"pad": "x" * 2000}} for m in range(1, 12)}
+    dec = {"per_m": per_m}
+    sections = {"per_m": per_m, "moe": None}
+    line = {"metric": bench.METRIC, "value": 1.0,
+            "summary": bench.headline_summary(dec, None, {"us": 127.98, "frac": 0.3577}, {"per_m": per_m}, None, None, None)}
+    out = bench.report(sections, line)
+    assert len(out) == 2 and out[0].startswith("# per_m: ") and len(out[0]) > 8192
+    assert json.loads(out[-1]) == line and len(out[-1]) < 4096 and "\n" not in out[-1]

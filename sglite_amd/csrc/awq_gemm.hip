@@ -10,8 +10,8 @@
 //    mfma32_kernel on 32x32x16 ones): prefill (MFMA-bound), mid-size batches
 //    and 5-32 rows on large or deep matrices, split K summed by a second
 //    reduction kernel (or, on request, inside the GEMM kernel);
-//  * ring_kernel (awq_ring.hip): in place of the tiled kind at 17-64 rows, where
-//    its cost model fits (plan_ring);
+//  * ring_kernel (awq_ring.hip): in place of most tiled plans at 17-64 rows
+//    (plan_ring);
 //  * kslice_kernel (awq_kslice.hip): decode batches up to 32 rows, split K
 //    reduced by the last workgroup of each column group (planner override
 //    only).
@@ -338,23 +338,33 @@ bool plan_kslice(const Geom& g, int v, int act, GemmPlan& p) {
 // 11.59).
 
 // ring_kernel (awq_ring.hip) in place of the tiled plan p at 17-64 rows.
-// (The GEMV and decode kernels' plans stay: those scale each group's sum in
-// fp32, where this kernel, like the tiled ones, rounds every weight.)
+// The GEMV and decode kernels' plans stay: the decode kernel, and the GEMV
+// kernel in fp16, scale each group's sum in fp32, where this kernel, like the
+// tiled ones, rounds every weight.  The GEMV kernel in bf16 rounds them too
+// from four rows; there the ring form would gain 0-5% on 2560 x 6144 and 4-10%
+// on 2560 x 19456 and 1024 x 8192, but one plan serves both types.
 //
 // Column tiles per workgroup (t) and k-slices (ks) come from a cost model
 // fitted to sweeps of every shape over the Qwen3-4B, Llama-3-8B and
 // tensor-parallel linears at M = 20 .. 64: us = a launch + k-tiles of a
 // workgroup x the time of one (more tiles cost dequantisation and MFMAs, more
-// rows activation traffic) + the partials' second kernel; a workgroup's ring
-// fills most of a CU's LDS, so the grid is at most one per CU.  Larger layers
-// (70B-sized qkv, gate_up and down, 1.1-1.3 times slower here) keep the tiled
-// plan, and so do more than 32 k-tiles a slice, the 64-row form with four
-// groups per k-tile (spills; 4096 x 2560 of G = 32 and deeper 1.1-1.6 times
-// slower) and its deep K with two (0.95-0.98).
-// Graph-replay A/B at M = 17-64 over 300 cases: 1.2 times faster on average
-// (Qwen3-4B qkv / o / gate_up / down at M = 32 fp16 11.4 -> 7.7 / 11.1 -> 7.9 /
-// 16.4 -> 12.7 / 12.5 -> 11.4 us; Llama-3-8B qkv / o / gate_up / down at
-// M = 64 14.9 -> 12.8 / 13.8 -> 11.4 / 33.1 -> 25.2 / 20.1 -> 19.8).
+// rows activation traffic) + the partials' second kernel.  The grid is at most
+// one workgroup per CU.  At 33-64 rows the ring takes 96 KiB of LDS or more, so
+// no second one fits; at 17-32 rows two of eight waves do, but grids of up to
+// 512 were faster by more than 2% in 10 of 171 measured (shape, rows, type)
+// cases, by 7% at most.  Larger layers (70B-sized qkv, gate_up and down, 1.1-1.3
+// times slower here) keep the tiled plan, and so do more than 32 k-tiles a
+// slice, the 64-row form with four groups per k-tile (spills; 4096 x 2560 of
+// G = 32 and deeper 1.1-1.6 times slower) and its deep K with two (0.95-0.98).
+// At 17-32 rows slices of 32 k-tiles keep it as well: 64 k-tiles in two slices
+// (8192 x 7168 gated, 8192 x 8192) lost 5-8% there in fp16 at 17-20 rows
+// (15.5 -> 16.8 us) and gained 4-11% in bf16 at 28-32.
+// Graph-replay A/B at M = 17-64 over 445 cases that the rule takes (25 layer
+// shapes, both types, G = 128, 64 and 32): 1.26 times faster on average, the
+// slowest 0.987 (Llama-3-8B down at M = 20, 15.1 -> 15.3 us).  Qwen3-4B qkv / o /
+// gate_up / down at M = 32 fp16 11.5 -> 8.2 / 10.9 -> 8.2 / 16.7 -> 13.4 / 12.7 ->
+// 11.3 us; Llama-3-8B at M = 64 15.7 -> 13.1 / 14.1 -> 11.9 / 34.8 -> 27.0 /
+// 20.7 -> 20.0.
 void plan_ring(const Geom& g, int act, GemmPlan& p) {
   const int forced = knob(kPlanRing, kUnset);
   if (forced == 0 || g.M < 17 || g.M > 64) return;
@@ -394,7 +404,7 @@ void plan_ring(const Geom& g, int act, GemmPlan& p) {
     for (int ks : {1, 2, 3, 4, 6, 8}) {
       if (ks > 1 && (t > 4 || ks * slice > p.ws_bytes || ks > g.KT / 4)) break;
       const int64_t ktc = (g.KT + ks - 1) / ks, kse = (g.KT + ktc - 1) / ktc;
-      if (cols * kse > g.cus || ktc > (kse > 1 && mt == 2 ? 31 : 32)) continue;
+      if (cols * kse > g.cus || ktc > (kse > 1 && mt == 2 ? 31 : 32)) continue;  // 31: see above
       double us = 3.2 + 0.2 * mt + (double)ktc * per_kt;
       if (kse > 1) us += 1.2 + 0.2 * mt + (double)(kse * slice) * 0.6e-6;
       if (best == 0.0 || us < best) {

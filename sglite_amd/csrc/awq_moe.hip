@@ -300,10 +300,13 @@ __global__ __launch_bounds__(kAlignThreads) void align_kernel(const int32_t* __r
 // Routing and alignment of a decode batch in one launch: each wave of one
 // workgroup routes a token and the same workgroup aligns the ids, which it
 // keeps in LDS.  A launch of a captured step costs about 1 us beyond its work,
-// so one token per wave is the line: a block of E = 128, H = 2048, I = 768
-// top-8 experts (fp16, whole forward) takes 26.5 us at T = 1 with it and 27.2
-// with two launches (28.4 with the logits' conversion a third), 74.3 and 73.8
-// at T = 16, 86.6 and 83.8 at T = 32, where the waves route two tokens in turn.
+// and 16 waves on one CU take longer over 16 tokens than 16 CUs do, so one token
+// per wave is the line.  Whole forwards of a block, one launch against two:
+// E = 128, H = 2048, I = 768 top-8 fp16 at T = 1 / 8 / 12 / 16 22.3 against 23.4 /
+// 50.6 against 51.6 / 56.5 against 57.0 / 62.5 against 62.4 us; E = 16, H = 1024
+// top-2 bf16 at T = 16 20.6 against 21.5; E = 512 top-8 24.5 against 25.4 at T = 1
+// and 67.0 against 65.6 at T = 16.  (Waves that routed two tokens in turn lost
+// 3% at T = 32.)
 constexpr int kRouteTokens = kAlignWaves;
 constexpr int kRouteRows = kRouteTokens * 64;  // the ids in LDS (at most 64 experts per token)
 
@@ -894,10 +897,12 @@ hipError_t launch_moe_gemm(const MoeGemmParams& p, hipStream_t s) {
   // grid is the blocks that have rows.  Here most experts are empty, and the
   // grid below, sized for every expert being busy, leaves the rest of a token's
   // 8 experts to 32 workgroups (E = 128, H = 2048, I = 768 top-8 fp16 / bf16, a
-  // block's whole forward: T = 1 56.7 -> 28.4 / 67.4 -> 29.2 us, T = 8 69.9 ->
-  // 58.5 / 82.6 -> 62.3, T = 16 81.5 -> 73.4 / 96.2 -> 78.5; beyond that line
-  // it loses: T = 32 84.7 -> 90.2, and E = 64, H = 2048, I = 1408 at T = 16
-  // 82.7 -> 83.4).  Its per-expert weight offsets are 32 bits, past-the-end
+  // block's whole forward: T = 1 55.0 -> 25.6 / 65.4 -> 26.4 us, T = 8 67.3 ->
+  // 55.1 / 82.3 -> 58.1, T = 16 74.4 -> 65.6 / 91.0 -> 71.7).  At the line every
+  // shape measured gains in both types; where it starts to lose depends on the
+  // type: in fp16 T = 20 70.6 -> 68.8, T = 24 71.2 -> 73.3, T = 32 72.5 -> 82.0,
+  // in bf16 T = 24 86.8 -> 77.6, T = 32 87.4 -> 86.6, T = 48 88.2 -> 99.2 (E = 64,
+  // H = 2048, I = 1408 fp16 at T = 16 71.6 -> 70.2, T = 24 73.6 -> 79.4).  Its per-expert weight offsets are 32 bits, past-the-end
   // offsets bit 31.
   if (p.num_routed <= p.E && p.g.NT * p.g.KT * 1024 < (int64_t(1) << 31)) return launch_moe_rows(p, s);
   MoeArgs a{};

@@ -94,9 +94,10 @@ struct Blocks {
 // workgroups many: four waves while the blocks are fewer than half the experts,
 // two beyond, where more resident workgroups hide the chain better (E = 128,
 // H = 2048, I = 768 top-8 fp16, a block's whole forward at T = 1 / 4 / 8 / 16:
-// four waves 28.4 / 46.4 / 62.9 / 84.5 us, two 30.2 / 43.8 / 58.5 / 73.4; four
-// tiles instead of two 29.3 / 45.0 / 59.2 / 76.8 at four waves; 56.7 / 59.3 /
-// 69.9 / 81.5 in the pipelined kernel).
+// four waves 25.6 / 39.7 / 55.1 / 76.6 us, two 27.6 / 37.1 / 50.5 / 65.6, and
+// 55.0 / 55.2 / 67.3 / 74.4 in the pipelined kernel: the two cross between 8 and
+// 32 rows here, below the line).  Four tiles at four waves cost 3% at T = 1, and
+// 5% at T = 16 against two at two.
 constexpr int kTiles = 2;
 constexpr int kMaxWaves = 4;
 

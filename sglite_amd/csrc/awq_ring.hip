@@ -7,20 +7,24 @@
 // k-tiles and the WN waves of a k-tile share its activations.  A step's
 // weights, zero points and scales (registers) and activations (LDS-DMA into
 // the ring) are in flight during the step before it.  The WK partial sums meet
-// in LDS at the end; K is mostly unsplit.
+// in LDS at the end.  K stays unsplit where the column tiles give enough
+// workgroups (qkv and gate_up of Qwen3-4B and Llama-3-8B); their o and down
+// leave K in 3 to 6 slices, summed by a second launch (3-5 us) as the tiled
+// plans' 4 to 16 are.
 //
 // What bounds these shapes is not the weight stream but the dequantisation,
 // LDS reads and MFMAs of a k-tile following one another: the tiled kernels put
-// four waves on a CU here, one per SIMD, and needed a second kernel for the K
-// slices that filled the chip.  With 8 to 16 waves on a CU the units overlap.
-// Measured against them (graph replay, us; floor at the copy rate of 4.8 TB/s
-// in brackets): Qwen3-4B at M = 32, fp16, qkv 11.4 -> 7.7 (1.7), o 11.1 -> 7.9
-// (1.1), gate_up 16.4 -> 12.7 (5.4), down 12.5 -> 11.4 (2.7); Llama-3-8B at
-// M = 64 qkv 14.9 -> 12.8 (2.7), o 13.8 -> 11.4 (1.8), gate_up 33.1 -> 25.2
-// (12.5), down 20.1 -> 19.8 (6.3).  Tried: four slots, three steps ahead, with
-// half the waves (gate_up at M = 64 27.6); four tiles per wave and half the
-// waves, which halves the LDS reads (26.0); one m-tile at M = 8, where the GEMV
-// and decode kernels stay ahead (qkv 5.9 against 5.7).
+// four waves on a CU here, one per SIMD.  With 8 to 16 waves on a CU the units
+// overlap.  Measured against them (graph replay, us; floor at the copy rate of
+// 4.8 TB/s in brackets): Qwen3-4B at M = 32, fp16, qkv 11.5 -> 8.2 (1.7), o
+// 10.9 -> 8.2 (1.1), gate_up 16.7 -> 13.4 (5.4), down 12.7 -> 11.3 (2.7);
+// Llama-3-8B at M = 64 qkv 15.7 -> 13.1 (2.7), o 14.1 -> 11.9 (1.8), gate_up
+// 34.8 -> 27.0 (12.5), down 20.7 -> 20.0 (6.3: alone on the device its GEMM is
+// a little longer than the tiled one, 17.9 against 16.6).  Tried: four slots,
+// three steps ahead, with half the waves (gate_up at M = 64 27.6 against 25.2);
+// four tiles per wave and half the waves, which halves the LDS reads (26.0
+// against 25.2); one m-tile at M = 8, where the GEMV and decode kernels stay
+// ahead (qkv 5.9 against 5.7).
 #include <algorithm>
 
 #include "awq_buffer.h"

@@ -1018,8 +1018,10 @@ hipError_t launch_bm(const TiledArgs& a, int gpt, hipStream_t s) {
 template <typename DT>
 hipError_t launch_dt(const GemmPlan& p, const TiledArgs& a, int gpt, hipStream_t s) {
   // The bf16 32-row form is cut for three workgroups per CU (141 registers):
-  // at four it would spill inside the loop (Qwen3-4B decode linears at M = 32:
-  // 77 us a layer with 57 spilled registers, 58.8 at three workgroups).
+  // at four it would spill inside the loop.  At the sizes it serves, three are
+  // 1-6% faster (9728 x 2560 at M = 16 / 72 / 112 12.8 -> 12.3 / 20.0 -> 19.6 /
+  // 23.1 -> 22.7 us, 4096 x 6144 at M = 96 / 160 21.4 -> 20.8 / 27.4 -> 27.0,
+  // 8192 x 10240 at M = 8 / 32 20.4 -> 19.3 / 22.1 -> 21.6).
   constexpr int kOcc32 = std::is_same_v<DT, BF16> ? 3 : 4;
   switch (p.variant) {
     case 32: return launch_bm<32, DT>(a, gpt, s);

@@ -1,11 +1,14 @@
-// Buffer-resource helpers and the 32x32x16 MFMA, shared by the MFMA GEMM
-// kernels (awq_tiled.hip, awq_kslice.hip).
+// Buffer-resource helpers, weight stages and the 32x32x16 MFMA, shared by the
+// MFMA GEMM kernels.
 #pragma once
 
 #include "awq_device.h"
 
 namespace sgl_awq {
 
+// Offset past every buffer range (the kernels that use it keep ranges below
+// 2^31): such a load returns zeros without a memory access.
+constexpr uint32_t kPastEnd = 0x80000000u;
 constexpr uint32_t kRsrcWord3 = 0x00020000u;  // raw buffer, dword data format (gfx9)
 // Buffer cache policy SC1 (device scope): the bits the compiler gives an
 // agent-scope atomic store; the store is written through the L2, so the
@@ -83,6 +86,62 @@ struct WStage32 {
   u32x4 q[2][2];       // [column group][even / odd k-step vector]
   uint32_t z[2][GPT];  // the zero-point word holding this lane's nibble, per quantisation group
   uint16_t s[2][GPT];  // this lane's column scale, per quantisation group
+};
+
+// The same in the 16x16x32 operand order for a wave's NTW column tiles: lane l
+// holds its column's words of the four k-blocks.
+template <int NTW, int GPT>
+struct WStage16 {
+  u32x4 q[NTW];
+  uint32_t z[NTW][GPT];  // zero-point word holding the lane's nibble
+  uint16_t s[NTW][GPT];  // scale bits
+
+  template <typename DT>
+  __device__ __forceinline__ void zero_scale(int lane, typename Dq<DT>::ZS (&zs)[NTW][GPT]) const {
+#pragma unroll
+    for (int gg = 0; gg < GPT; ++gg)
+#pragma unroll
+      for (int j = 0; j < NTW; ++j) zs[j][gg] = Dq<DT>::make((z[j][gg] >> (4 * (lane & 7))) & 0xFu, s[j][gg]);
+  }
+};
+
+// Where a wave's column tiles come from: the matrix's weights, zeros and
+// scales as buffer ranges, and the wave's tiles in them.
+template <int NTW, int GPT>
+struct WTiles {
+  static constexpr int BPG = 4 / GPT;  // k-blocks per quantisation group
+  __amdgpu_buffer_rsrc_t wr, zr, sr;
+  uint32_t tile[NTW];
+  uint32_t past[NTW];  // kPastEnd for a tile the matrix does not have, else 0
+  int KT, NG, gshift;
+
+  __device__ __forceinline__ void set_matrix(const void* w, const void* s, const void* z, int NT) {
+    wr = make_rsrc(w, (uint32_t)NT * (uint32_t)KT * 1024u);
+    zr = make_rsrc(z, (uint32_t)NT * (uint32_t)NG * 8u);
+    sr = make_rsrc(s, (uint32_t)NT * (uint32_t)NG * 32u);
+  }
+  __device__ __forceinline__ void set_tile(int j, int nt, bool in) {
+    tile[j] = in ? (uint32_t)nt : 0u;
+    past[j] = in ? 0u : kPastEnd;
+  }
+  // k-tile kt; `dead` kPastEnd (past the wave's range) loads zeros.
+  __device__ __forceinline__ void load(WStage16<NTW, GPT>& st, int kt, uint32_t dead, int lane) const {
+    const uint32_t wo = (uint32_t)lane * 16u | dead;
+    const uint32_t zo = (uint32_t)((lane & 15) >> 3) * 4u | dead;
+    const uint32_t so = (uint32_t)(lane & 15) * 2u | dead;
+#pragma unroll
+    for (int j = 0; j < NTW; ++j)
+      st.q[j] = __builtin_amdgcn_raw_buffer_load_b128(wr, wo | past[j], (tile[j] * KT + kt) * 1024, kCacheStream);
+#pragma unroll
+    for (int gg = 0; gg < GPT; ++gg) {
+      const int g = min((kt * 128 + 32 * BPG * gg) >> gshift, NG - 1);
+#pragma unroll
+      for (int j = 0; j < NTW; ++j) {
+        st.z[j][gg] = __builtin_amdgcn_raw_buffer_load_b32(zr, zo | past[j], (tile[j] * NG + g) * 8, 0);
+        st.s[j][gg] = __builtin_amdgcn_raw_buffer_load_b16(sr, so | past[j], (tile[j] * NG + g) * 32, 0);
+      }
+    }
+  }
 };
 
 }  // namespace sgl_awq

@@ -135,29 +135,29 @@ __global__ __launch_bounds__(64 * kMaxWaves, GPT < 4 && EPL <= 2 ? 4 : 3) void m
     if (__ballot(valid) == 0) continue;
     const float rw = a.mul_rw && valid ? a.topk_w[sid] : 1.f;
 
-    KWave<1, NTW, GPT, DT> kw;
-    kw.K = a.K;
-    kw.KT = a.KT;
-    kw.NG = a.NG;
-    kw.gshift = a.gshift;
-    kw.lane = lane;
-    kw.dk = dq_consts();
-    kw.xr = make_rsrc(a.x, a.x_bytes);
-    kw.xoff[0] = valid ? (uint32_t)(sid / a.a_div) * (uint32_t)a.K * 2u + (uint32_t)(lane >> 4) * 16u : kPastEnd;
-    kw.set_matrix(a.wt + e * a.w_stride, a.s_r + e * a.s_stride, a.z_r + e * a.z_stride, a.NT);
+    KWave<NTW, GPT, DT> kw;
+    kw.w.KT = a.KT;
+    kw.w.NG = a.NG;
+    kw.w.gshift = a.gshift;
+    kw.w.set_matrix(a.wt + e * a.w_stride, a.s_r + e * a.s_stride, a.z_r + e * a.z_stride, a.NT);
     const int half = ACT == kActNone ? a.NT : a.NT >> 1;
 #pragma unroll
     for (int j = 0; j < NTW; ++j) {
       const int t = tile0 + j % HT;
-      kw.set_tile(j, t + j / HT * half, t < half);
+      kw.w.set_tile(j, t + j / HT * half, t < half);
     }
-    f32x4 acc[1][NTW];
+    kw.K = a.K;
+    kw.lane = lane;
+    kw.dk = dq_consts();
+    kw.xr = make_rsrc(a.x, a.x_bytes);
+    kw.xoff = valid ? (uint32_t)(sid / a.a_div) * (uint32_t)a.K * 2u + (uint32_t)(lane >> 4) * 16u : kPastEnd;
+    f32x4 acc[NTW];
 #pragma unroll
-    for (int j = 0; j < NTW; ++j) acc[0][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NTW; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
     kw.template run<2>(kt0, kt1, acc);
 
 #pragma unroll
-    for (int j = 0; j < NTW; ++j) red[wave * NQ + j * 64 + lane] = acc[0][j];
+    for (int j = 0; j < NTW; ++j) red[wave * NQ + j * 64 + lane] = acc[j];
     __syncthreads();
     // Wave w sums and stores tiles w, w + WK, ... of the group: lane (c, lg)
     // holds row c of the block and columns 4 lg .. 4 lg + 3.

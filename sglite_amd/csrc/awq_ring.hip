@@ -36,7 +36,6 @@ namespace sgl_awq {
 namespace {
 
 constexpr int kRingLds = 160 * 1024;
-constexpr uint32_t kPastEnd = 0x80000000u;  // past every buffer range (below 2^31): such a load returns zeros
 
 struct RingArgs {
   const void* x;
@@ -59,7 +58,6 @@ template <int MT, int NTW, int NX, int GPT, typename DT>
 __global__ __launch_bounds__(1024, 4) void ring_kernel(RingArgs a) {
   using E = typename DT::elem;
   using V8 = typename DT::vec8;
-  constexpr int BPG = 4 / GPT;
   constexpr int XT = MT * 256;  // 16-byte vectors of one k-tile's activations
   extern __shared__ u32x4 ring[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -69,22 +67,21 @@ __global__ __launch_bounds__(1024, 4) void ring_kernel(RingArgs a) {
   const bool paired = a.act != kActNone;
   const int half = a.NT >> 1;
   constexpr int HT = NTW > 1 ? NTW / 2 : 1;  // gate tiles of a wave with a gated activation
-  uint32_t tile[NTW], past[NTW];
+  WTiles<NTW, GPT> wt;
+  wt.KT = a.KT;
+  wt.NG = a.NG;
+  wt.gshift = a.gshift;
+  wt.set_matrix(a.w, a.s, a.z, a.NT);
 #pragma unroll
   for (int j = 0; j < NTW; ++j) {
     const int t = paired ? (blockIdx.x * WN + wn) * HT + j % HT + j / HT * half : (blockIdx.x * WN + wn) * NTW + j;
-    const bool in = t < (paired ? half + j / HT * half : a.NT);
-    tile[j] = in ? (uint32_t)t : 0u;
-    past[j] = in ? 0u : kPastEnd;
+    wt.set_tile(j, t, t < (paired ? half + j / HT * half : a.NT));
   }
   const int kt_begin = blockIdx.y * a.ktc, kt_end = min(kt_begin + a.ktc, a.KT);
   const int steps = (kt_end - kt_begin + WK - 1) / WK;
   const DqK dk = dq_consts();
 
   const __amdgpu_buffer_rsrc_t xr = make_rsrc(a.x, (uint32_t)a.M * (uint32_t)a.K * 2u);
-  const __amdgpu_buffer_rsrc_t wr = make_rsrc(a.w, (uint32_t)a.NT * (uint32_t)a.KT * 1024u);
-  const __amdgpu_buffer_rsrc_t zr = make_rsrc(a.z, (uint32_t)a.NT * (uint32_t)a.NG * 8u);
-  const __amdgpu_buffer_rsrc_t sr = make_rsrc(a.s, (uint32_t)a.NT * (uint32_t)a.NG * 32u);
 
   // The wave's share of its k-tile's activations: NX groups of four rows (a
   // group past the last repeats it, so that every wave counts NX loads).
@@ -100,11 +97,7 @@ __global__ __launch_bounds__(1024, 4) void ring_kernel(RingArgs a) {
     xdst[i] = rg * 64;
   }
 
-  struct Stage {
-    u32x4 q[NTW];
-    uint32_t z[NTW][GPT];
-    uint16_t s[NTW][GPT];
-  };
+  using Stage = WStage16<NTW, GPT>;
   // Step i's loads in the order the wait counts rely on: activations, weights.
   auto issue = [&](Stage& st, int i, int slot) {
     const int kt = kt_begin + i * WK + kw;
@@ -116,21 +109,7 @@ __global__ __launch_bounds__(1024, 4) void ring_kernel(RingArgs a) {
       load_lds16(xr, dst + xdst[n], off, kt * 256);
     }
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = 0; j < NTW; ++j)
-      st.q[j] = __builtin_amdgcn_raw_buffer_load_b128(wr, (uint32_t)lane * 16u | dead | past[j],
-                                                      (tile[j] * a.KT + kt) * 1024, kCacheStream);
-#pragma unroll
-    for (int gg = 0; gg < GPT; ++gg) {
-      const int g = min((kt * 128 + 32 * BPG * gg) >> a.gshift, a.NG - 1);
-#pragma unroll
-      for (int j = 0; j < NTW; ++j) {
-        st.z[j][gg] = __builtin_amdgcn_raw_buffer_load_b32(zr, (uint32_t)(c >> 3) * 4u | dead | past[j],
-                                                           (tile[j] * a.NG + g) * 8, 0);
-        st.s[j][gg] = __builtin_amdgcn_raw_buffer_load_b16(sr, (uint32_t)c * 2u | dead | past[j],
-                                                           (tile[j] * a.NG + g) * 32, 0);
-      }
-    }
+    wt.load(st, kt, dead, lane);
     __builtin_amdgcn_sched_barrier(0);
   };
 
@@ -142,10 +121,7 @@ __global__ __launch_bounds__(1024, 4) void ring_kernel(RingArgs a) {
 
   auto mul = [&](const Stage& st, const u32x4* xs) {
     typename Dq<DT>::ZS zs[NTW][GPT];
-#pragma unroll
-    for (int gg = 0; gg < GPT; ++gg)
-#pragma unroll
-      for (int j = 0; j < NTW; ++j) zs[j][gg] = Dq<DT>::make((st.z[j][gg] >> (4 * (c & 7))) & 0xFu, st.s[j][gg]);
+    st.template zero_scale<DT>(lane, zs);
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       V8 b[MT];
@@ -154,7 +130,7 @@ __global__ __launch_bounds__(1024, 4) void ring_kernel(RingArgs a) {
       for (int mt = 0; mt < MT; ++mt) b[mt] = __builtin_bit_cast(V8, xs[mt * 256 + at]);
 #pragma unroll
       for (int j = 0; j < NTW; ++j) {
-        const V8 v = Dq<DT>::word(st.q[j][w], zs[j][w / BPG], dk);
+        const V8 v = Dq<DT>::word(st.q[j][w], zs[j][w / wt.BPG], dk);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[mt][j] = mfma16x16x32(v, b[mt], acc[mt][j]);
       }

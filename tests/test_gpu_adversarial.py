@@ -96,6 +96,18 @@ def test_tiled_dequant_path(dtype, kind):
 
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("dtype", DTYPES)
+def test_ring_and_tiled_kernels_at_48_rows(dtype, kind, plan):
+    """Of that plan kind ring_kernel runs there; the prefill kernel itself without it."""
+    from sglite_amd import ops
+
+    assert ops.launch_info(48, 1024, 4096, 128).function == "ring_kernel"
+    plan.set("ring", 0)
+    assert ops.launch_info(48, 1024, 4096, 128).function in ("tiled_kernel", "mfma32_kernel")
+    _run(48, 4096, 1024, dtype, kind, kernel="tiled_kernel")
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("M", [8, 32])
 def test_kslice_dequant_path(M, dtype, kind, plan):
     """The k-slice decode kernel (bit-exact dequantisation into 32x32 MFMAs, the split-K

@@ -70,6 +70,14 @@ def test_fused_silu_matches_oracle(M, K, I, kernel, dtype, plan):
     _check(M, K, I, dtype=dtype, kernel=kernel, plan=plan)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_fused_silu_on_the_tiled_plan_of_40_rows(dtype, plan):
+    """The split-K tiled plan above, where ring_kernel runs in its place."""
+    assert _ops().launch_info(40, 2080, 2048, 128, "silu").function == "ring_kernel"
+    _check(40, 2048, 1040, dtype=dtype, kernel="tiled_kernel", env={"ring": 0}, plan=plan)
+    assert _ops().launch_info(40, 2080, 2048, 128, "silu").function in ("tiled_kernel", "mfma32_kernel")
+
+
 @pytest.mark.parametrize("M", [7, 8])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("with_bias", [False, True])

@@ -502,6 +502,19 @@ def test_tiled_split_k_parity_and_determinism(M, K, N, G):
     workgroups; a second kernel sums the slices' fp32 partials in slice
     order, so repeated calls and graph replays are bit-identical, and the
     counters are left at zero."""
+    _split_k_parity_and_determinism(M, K, N, G)
+
+
+@pytest.mark.parametrize("M,K,N,G", [(64, 14336, 4096, 128), (40, 2368, 264, 32), (24, 4096, 28672, 128)])
+def test_split_k_parity_of_the_tiled_plans_at_17_to_64_rows(M, K, N, G, plan):
+    """The shapes of the test above that launch ring_kernel, on the plan it takes the place of."""
+    assert _ops().launch_info(M, N, K, G).function == "ring_kernel"
+    plan.set("ring", 0)
+    assert _ops().launch_info(M, N, K, G).function in ("tiled_kernel", "mfma32_kernel")
+    _split_k_parity_and_determinism(M, K, N, G)
+
+
+def _split_k_parity_and_determinism(M, K, N, G):
     ops = _ops()
     assert ops.gemm_kernel(M, N, K, G) == "tiled_kernel"
     assert ops.workspace_bytes(M, N, K, G) > 0

@@ -51,6 +51,25 @@ def _cases(n=48, seed=77):
 
 @pytest.mark.parametrize("case", _cases(), ids=lambda c: f"c{c[0]}-M{c[1]}-K{c[2]}-N{c[3]}-G{c[4]}")
 def test_split_k_tail_steps_read_landed_activations(case):
+    _run(case)
+
+
+def _on_ring(case):
+    from sglite_amd import ops
+
+    return ops.launch_info(case[1], case[3], case[2], case[4]).function == "ring_kernel"
+
+
+@pytest.mark.parametrize("case", [c for c in _cases() if _on_ring(c)],
+                         ids=lambda c: f"c{c[0]}-M{c[1]}-K{c[2]}-N{c[3]}-G{c[4]}")
+def test_the_same_on_the_tiled_kernels(case, plan):
+    """The cases of 17-64 rows that launch ring_kernel, on the plan it takes the place of."""
+    plan.set("ring", 0)
+    assert not _on_ring(case)
+    _run(case)
+
+
+def _run(case):
     from sglite_amd import ops
 
     i, M, K, N, G, dtype = case

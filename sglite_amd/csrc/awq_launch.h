@@ -141,7 +141,10 @@ struct MoeGemmParams {
   int dtype;
 };
 hipError_t launch_moe_gemm(const MoeGemmParams& p, hipStream_t s);
-// The form for few routed rows per expert (awq_moe_rows.hip).
+// The form for few routed rows per expert (awq_moe_rows.hip): its waves per
+// workgroup and column-tile groups.
+int moe_rows_waves(const MoeGemmParams& p);
+int64_t moe_rows_groups(const MoeGemmParams& p);
 hipError_t launch_moe_rows(const MoeGemmParams& p, hipStream_t s);
 // Streaming probe (awq_probe.hip).
 hipError_t launch_stream_probe(const void* src, int64_t bytes, int64_t grid, int block, uint32_t* sink,

@@ -806,11 +806,14 @@ __global__ __launch_bounds__(256) void moe_sum_kernel(const typename DT::elem* _
   *(V8*)(out + t * H + n0) = r;
 }
 
+// Weight k-tiles in registers (NS) for a shape.
+int weight_stages(int gpt, int KT) { return gpt >= 4 ? 2 : gpt == 2 ? 3 : KT % 4 != 0 && KT % 3 == 0 ? 3 : 4; }
+
 template <typename DT>
 hipError_t launch_moe_gemm_dt(const MoeArgs& a, int tw, int gpt, int epi, int passes, hipStream_t s) {
   const int64_t gx = (a.total + 7) / 8 * 8;
   dim3 grid((unsigned)gx, (unsigned)passes);
-  const int ns = gpt >= 4 ? 2 : gpt == 2 ? 3 : (a.KT % 4 != 0 && a.KT % 3 == 0) ? 3 : 4;
+  const int ns = weight_stages(gpt, a.KT);
 #define SGL_MOE(TW_, GPT_, EPI_, NS_)                                                                \
   if (tw == TW_ && gpt == GPT_ && epi == EPI_ && ns == NS_) {                                        \
     hipLaunchKernelGGL((moe_gemm_kernel<TW_, GPT_, EPI_, NS_, DT>), grid, dim3(kThreads), 0, s, a);  \
@@ -892,19 +895,51 @@ hipError_t launch_moe_align(const int32_t* ids, int64_t n, int64_t E, int64_t bs
   return hipGetLastError();
 }
 
+namespace {
+
+// The row-block form (awq_moe_rows.hip) or the pipelined one below for a GEMM
+// whose pipelined workgroups take U slices each.
+//
+// With at most one routed row per expert on average most experts are empty or
+// hold a row or two.  The pipelined grid is sized for every expert being busy
+// and leaves the rest of a token's 8 experts to 32 workgroups; the row-block
+// grid is as large as the work (E = 128, H = 2048, I = 768 top-8 fp16 / bf16, a
+// block's whole forward: T = 1 55.0 -> 25.6 / 65.4 -> 26.4 us, T = 8 67.3 -> 55.1 /
+// 82.3 -> 58.1, T = 16 74.4 -> 65.6 / 91.0 -> 71.7).  At one row per expert every
+// shape like these still gains in both types; where it starts to lose depends on
+// the type: in fp16 T = 20 70.6 -> 68.8, T = 24 71.2 -> 73.3, T = 32 72.5 -> 82.0,
+// in bf16 T = 24 86.8 -> 77.6, T = 32 87.4 -> 86.6, T = 48 88.2 -> 99.2.
+//
+// Below that line the row-block form loses where its workgroups are many and
+// short (many experts, few k-tiles): each pays its chain of offsets, rows,
+// weights and sum for a k-tile or two per wave, while a pipelined workgroup pays
+// it once.  So its waves per CU, in rounds of the 16 that a CU holds, are set
+// against the pipelined workgroups' k-steps.  The weights come from GEMMs of
+// both forms over 24-512 experts, K = 128 .. 2048, N = 512 .. 4096, n = 4 .. E, all
+// group sizes and both types (3483 cases): more than 128 experts make a round
+// longer (the scan), so do two or four groups per k-tile and four waves (their
+// sum), and the pipelined form's dequantisation is longer in bf16.  With it the
+// GEMMs are 1.58 times faster than in the pipelined form on average and 19 of
+// them more than 5% slower (13% at most); with the row-block form throughout
+// 574 were, by up to three times.  E = 512, K = 512, N = 2048 at 256 rows 92.6 ->
+// 40.0 us, E = 128, K = 256, N = 1024, G = 32 at 64 rows 11.3 -> 8.2.
+bool rows_form(const MoeGemmParams& p, int gpt, int U, int64_t cus) {
+  // (Per-expert weight offsets of 32 bits, past-the-end offsets bit 31.)
+  if (p.num_routed > p.E || p.g.NT * p.g.KT * 1024 >= (int64_t(1) << 31)) return false;
+  const int ns = weight_stages(gpt, (int)p.g.KT);
+  const int64_t steps = U * ((p.g.KT + ns - 1) / ns * ns);
+  const int waves = moe_rows_waves(p);
+  double rounds = (double)moe_rows_groups(p) * (double)p.num_routed * waves / (16.0 * (double)cus);
+  if (p.E > 128) rounds *= 1.75;
+  if (gpt > 1) rounds *= 1.25;
+  if (waves > 2) rounds *= 1.25;
+  if (p.dtype != 0) rounds *= 0.65;
+  return rounds <= 0.35 * (double)steps;
+}
+
+}  // namespace
+
 hipError_t launch_moe_gemm(const MoeGemmParams& p, hipStream_t s) {
-  // At most one routed row per expert on average: the row-block form, whose
-  // grid is the blocks that have rows.  Here most experts are empty, and the
-  // grid below, sized for every expert being busy, leaves the rest of a token's
-  // 8 experts to 32 workgroups (E = 128, H = 2048, I = 768 top-8 fp16 / bf16, a
-  // block's whole forward: T = 1 55.0 -> 25.6 / 65.4 -> 26.4 us, T = 8 67.3 ->
-  // 55.1 / 82.3 -> 58.1, T = 16 74.4 -> 65.6 / 91.0 -> 71.7).  At the line every
-  // shape measured gains in both types; where it starts to lose depends on the
-  // type: in fp16 T = 20 70.6 -> 68.8, T = 24 71.2 -> 73.3, T = 32 72.5 -> 82.0,
-  // in bf16 T = 24 86.8 -> 77.6, T = 32 87.4 -> 86.6, T = 48 88.2 -> 99.2 (E = 64,
-  // H = 2048, I = 1408 fp16 at T = 16 71.6 -> 70.2, T = 24 73.6 -> 79.4).  Its per-expert weight offsets are 32 bits, past-the-end
-  // offsets bit 31.
-  if (p.num_routed <= p.E && p.g.NT * p.g.KT * 1024 < (int64_t(1) << 31)) return launch_moe_rows(p, s);
   MoeArgs a{};
   a.x = p.x;
   a.x_bytes = (uint32_t)((p.num_routed + p.a_div - 1) / p.a_div * p.g.K * 2);
@@ -942,6 +977,7 @@ hipError_t launch_moe_gemm(const MoeGemmParams& p, hipStream_t s) {
   const int64_t units_total = (int64_t)a.S * p.E * passes;
   const int64_t cus = device_cu_count();
   a.U = (int)std::min<int64_t>(std::max<int64_t>((units_total + 2 * cus - 1) / (2 * cus), 1), a.S);
+  if (rows_form(p, gpt, a.U, cus)) return launch_moe_rows(p, s);
   a.cpx = (int)std::max<int64_t>(cus / 8, 1);
   a.SG = (a.S + a.U - 1) / a.U;
   a.total = a.SG * (int)p.E;

@@ -36,6 +36,8 @@ struct RowsArgs {
   int mul_rw;
 };
 
+typedef int i32x4u __attribute__((ext_vector_type(4), aligned(4)));  // four offsets, aligned as one
+
 // The 16-row blocks of the experts' buckets, counted over the experts in
 // order.  One lane per EPL (2 or 8) experts; every wave of a workgroup finds
 // its blocks by itself.
@@ -46,8 +48,23 @@ struct Blocks {
 
   __device__ __forceinline__ void scan(const RowsArgs& a, int lane) {
     int o[EPL + 1];
+    if (EPL % 4 == 0 && a.E % EPL == 0) {
+      // Vectors of the lanes' own experts (lanes past the last expert reload
+      // the last ones'): nine loads of 32-byte stride a lane cost a CU whose 16
+      // waves all look for their blocks about 1 us (E = 512, K = 1024, N = 512
+      // gated at 256 rows 30.6 -> 22.8 us).
+      const int e0 = min(lane * EPL, a.E - EPL);
 #pragma unroll
-    for (int i = 0; i <= EPL; ++i) o[i] = a.offsets[min(lane * EPL + i, a.E)];
+      for (int i = 0; i < EPL / 4; ++i) {
+        const i32x4u v = *(const i32x4u*)(a.offsets + e0 + 4 * i);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) o[4 * i + k] = v[k];
+      }
+      o[EPL] = a.offsets[e0 + EPL];
+    } else {
+#pragma unroll
+      for (int i = 0; i <= EPL; ++i) o[i] = a.offsets[min(lane * EPL + i, a.E)];
+    }
     int sum = 0;
 #pragma unroll
     for (int i = 0; i < EPL; ++i) {
@@ -210,6 +227,13 @@ hipError_t launch_rows(const RowsArgs& a, int gpt, int act, dim3 grid, int waves
 
 }  // namespace
 
+int moe_rows_waves(const MoeGemmParams& p) { return 2 * p.num_routed > p.E ? 2 : kMaxWaves; }
+
+int64_t moe_rows_groups(const MoeGemmParams& p) {
+  const int64_t ht = p.epi ? kTiles / 2 : kTiles, cols = p.epi ? p.g.NT / 2 : p.g.NT;
+  return (cols + ht - 1) / ht;
+}
+
 hipError_t launch_moe_rows(const MoeGemmParams& p, hipStream_t s) {
   RowsArgs a{};
   a.x = p.x;
@@ -237,10 +261,9 @@ hipError_t launch_moe_rows(const MoeGemmParams& p, hipStream_t s) {
   a.z_stride = st.z / 8;
   a.mul_rw = p.mul_rw;
   const int gpt = (p.g.NG > 1 && p.g.G < 128) ? (int)(128 / p.g.G) : 1;
-  const int waves = 2 * p.num_routed > p.E ? 2 : kMaxWaves;
-  const int64_t ht = p.epi ? kTiles / 2 : kTiles, cols = p.epi ? p.g.NT / 2 : p.g.NT;
+  const int waves = moe_rows_waves(p);
   // At most one block with rows per routed row; each block of a table padded to 16 rows has one.
-  const dim3 grid((unsigned)((cols + ht - 1) / ht), (unsigned)p.num_routed);
+  const dim3 grid((unsigned)moe_rows_groups(p), (unsigned)p.num_routed);
 #define SGL_EPL(N_)                                                               \
   (p.dtype == 0 ? launch_rows<N_, F16>(a, gpt, p.epi, grid, waves, s)             \
                 : launch_rows<N_, BF16>(a, gpt, p.epi, grid, waves, s))

@@ -27,6 +27,9 @@ CASES = [  # (T, E, k, K, N, G, block size, routing)
     (2, 512, 4, 256, 64, 128, 16, "last"),      # the last expert
     (1, 4, 1, 256, 64, 128, 1024, "spread"),    # 63 blocks of padding behind one row, one workgroup per column group
     (5, 130, 7, 256, 64, 128, 256, "spread"),   # padding blocks dealt to every workgroup
+    (6, 136, 20, 256, 96, 64, 16, "last"),      # eight experts a lane as vectors, the last lanes without any
+    (2, 128, 8, 256, 1024, 32, 16, "spread"),   # short K: below the row-block form's line, ...
+    (8, 128, 8, 256, 1024, 32, 16, "spread"),   # ... and above it: the pipelined form
 ]
 
 
